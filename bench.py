@@ -170,7 +170,7 @@ def bench_mixed(prob, args, nnz, ms_fp64, variant, rows_z):
     a64, b64 = values()
     forms = {}
     prob.set_kernel(2)
-    forms["direct-store"] = (timed(), 2, 0)
+    forms["pair-lattice"] = (timed(), 2, 0)
     best = None
     for rz in (16, 32, 64):
         prob.set_kernel(0, rz)
@@ -651,7 +651,7 @@ def bench_batched(args):
            "ms_eager_one_by_one": round(ms_eager, 4), "speedup_graph_vs_eager": round(ms_eager / ms_graph, 3),
            "kernel_chosen_q1": {"z-marching 16": int((chosen == 16).sum()), "z-marching 32": int((chosen == 32).sum()),
                                 "z-marching 64": int((chosen == 64).sum()), "per-tile": int((chosen == -1).sum()),
-                                "per-tile direct-store": int((chosen == -2).sum()),
+                                "pair-lattice": int((chosen == -2).sum()),
                                 "per-tile wave-slab": int((chosen == -3).sum())}}
     out = {
         "metric": "batched assembly Gnnz/s (FP64), 32 Q1 problems" + ("" if el is None else " + elasticity Q2") +
@@ -737,14 +737,14 @@ def main():
     prob.symbolic()  # again on the same problem: the phase alone, past first-call set-up
     t_symbolic_again = time.perf_counter() - t0
     nnz = prob.owned_nnz()
-    # autotuner: z-marching columns of 16/32/64 rows, the per-tile kernel or its direct-store / wave-slab forms
+    # autotuner: the fastest form of the matrix kernel
     tuner = G.AssemblyBatch(ctx)
     tuner.add(prob)
     chosen = int(tuner.autotune(reps=3)[0])
     tuner.close()
     variant, rows_z = prob.get_kernel()
     kernel = {0: f"k_march3d<2,3,4,8> ({rows_z} z rows per workgroup)", 1: "k_assemble3d<2,3,4,8,8>",
-              2: "k_assemble3d_direct<2,3,4,8,8>", 3: "k_assemble3d_wslab<3,8>"}[variant]
+              2: "k_lattice (4 x 4 x 2 cells)", 3: "k_assemble3d_wslab<3,8>"}[variant]
 
     for _ in range(args.warmup):
         prob.numeric()
@@ -770,7 +770,7 @@ def main():
     # HBM bytes per launch measured with rocprofv3 FETCH_SIZE / WRITE_SIZE passes
     # (copy-calibrated) on this workload; only valid at the default size
     traffic = None
-    tname = {0: "k_march3d", 1: "k_assemble3d", 2: "k_assemble3d_direct", 3: "k_assemble3d_wslab"}[variant]
+    tname = {0: "k_march3d", 1: "k_assemble3d", 2: "k_lattice", 3: "k_assemble3d_wslab"}[variant]
     tpath = os.path.join(ROOT, "profiles", f"traffic_{tname}_poisson3d_q2_64.json")
     if args.cells == 64 and os.path.exists(tpath):
         with open(tpath) as fh:
@@ -796,7 +796,7 @@ def main():
             "parts": 8,
             "symbolic_s": round(t_symbolic, 3),
             "symbolic_s_again": round(t_symbolic_again, 4),
-            "autotuned": {"variant": {0: "z-marching", 1: "per-tile", 2: "per-tile direct-store",
+            "autotuned": {"variant": {0: "z-marching", 1: "per-tile", 2: "pair-lattice",
                                       3: "per-tile wave-slab"}[variant],
                           "z_rows_per_workgroup": rows_z},
             "mixed_fp32": mixed,

@@ -136,7 +136,6 @@ void order_tiles(gdx_problem *p) {
   const int cap = p->hbm_patterns       ? -1
                   : p->D != 3             ? 0
                   : p->kvariant3d == 1 ? gdx::pattern_capacity_tile3d(p->K, p->NQ)
-                  : p->kvariant3d == 2 ? gdx::pattern_capacity_tile3d_direct(p->K, p->NQ)
                   : p->kvariant3d == 3 ? gdx::pattern_capacity_tile3d_wslab(p->K, p->NQ)
                                        : gdx::pattern_capacity_3d(p->K, p->NQ);
   // (a tile without free rows has no pattern list to read from HBM: it stays in
@@ -232,6 +231,7 @@ void release_problem_device(gdx_problem *p) {
   gdx::flux_free(p);
   gdx::elast_free(p);
   gdx::mapped_free(p);
+  gdx::lattice_free(p);
   gdx::pvector_release(p);
   free_device(p);
   for (hipEvent_t &e : p->ev)
@@ -316,6 +316,7 @@ int gdx_symbolic(gdx_problem *p) {
     gdx::solve_free(p);  // its row tables are rebuilt from the new structure
     gdx::elast_free(p);
     gdx::flux_free(p);
+    gdx::lattice_free(p);
   }
   try {
     int rc = gdx::symbolic(p);
@@ -328,6 +329,7 @@ int gdx_symbolic(gdx_problem *p) {
     return GDX_ERR_ARG;
   }
   gdx::fill_kparams(p);
+  if (p->desc.op_kind == GDX_OP_DIFFUSION && gdx::lattice_used(p)) gdx::lattice_shape(p->D, p->K, p->tileR);
   order_tiles(p);
   if (!p->ctx) {
     p->symbolic_done = true;
@@ -335,11 +337,9 @@ int gdx_symbolic(gdx_problem *p) {
   }
   gdx::Device &d = p->dev;
   const bool elast = p->desc.op_kind == GDX_OP_ELASTICITY;
-  // kappa and f at the quadrature points (constant-coefficient elasticity has none)
-  const size_t nq = elast ? 1 : (size_t)p->kp.qn[0] * p->kp.qn[1] * p->kp.qn[2];
   int qnmax = std::max(p->kp.qn[0], std::max(p->kp.qn[1], p->kp.qn[2]));
-  GDX_HIP(gdx::dev_malloc(reinterpret_cast<void **>(&d.W), nq * sizeof(double)));
-  GDX_HIP(gdx::dev_malloc(reinterpret_cast<void **>(&d.F), nq * sizeof(double)));
+  if (p->desc.op_kind == GDX_OP_DIFFUSION)
+    if (int rp = gdx::points_alloc(p)) return rp;
   if (p->desc.nmodes > 0) {
     GDX_HIP(gdx::dev_malloc(reinterpret_cast<void **>(&d.E), (size_t)2 * 3 * p->desc.nmodes * qnmax * sizeof(double)));
     int rc = upload(&d.modes, p->modes);
@@ -363,6 +363,10 @@ int gdx_symbolic(gdx_problem *p) {
   if (!p->dev_structure && (rc = upload(&d.tile_pats, p->tile_pats))) return rc;
   if (elast && (rc = gdx::elast_setup(p))) {
     set_error("uploading the elasticity tables failed");
+    return rc;
+  }
+  if (p->desc.op_kind == GDX_OP_DIFFUSION && (rc = gdx::lattice_setup(p))) {
+    set_error("uploading the pair-lattice tables failed");
     return rc;
   }
   // the flux operator's lattice state and id map, set up here so that no
@@ -398,13 +402,45 @@ int retile(gdx_problem *p, const int R[3]) {
   return GDX_OK;
 }
 
+bool lattice_used(const gdx_problem *p) { return p->D == 2 || p->kvariant3d == 2; }
+
+// the tile kernels always read kappa and f at the points; the pair-lattice
+// kernel reads them only where kappa varies inside a cell
+int points_alloc(gdx_problem *p) {
+  if (p->dev.W || (lattice_used(p) && p->kp.nmodes == 0)) return GDX_OK;
+  const size_t nq = (size_t)p->kp.qn[0] * p->kp.qn[1] * p->kp.qn[2];
+  if (dev_malloc(&p->dev.W, nq * sizeof(double)) != hipSuccess ||
+      dev_malloc(&p->dev.F, nq * sizeof(double)) != hipSuccess) {
+    if (p->dev.W) (void)hipFree(p->dev.W);
+    p->dev.W = nullptr;
+    set_error("device allocation failed for the quadrature-point coefficients");
+    return GDX_ERR_ALLOC;
+  }
+  return GDX_OK;
+}
+
 // 3D kernel variant: 0 = z-marching columns with rows_z z rows per workgroup,
-// 1 = per-tile kernel, 2 = per-tile direct-store kernel, 3 = per-tile
-// wave-slab kernel (Q2 only); 1-3 use their own tile shape (rows_z ignored)
+// 1 = per-tile kernel, 2 = pair-lattice kernel, 3 = per-tile wave-slab kernel
+// (Q2 only); 1-3 use their own tile shape (rows_z ignored)
 int set_kernel_variant(gdx_problem *p, int variant, int rows_z) {
   if (p->D != 3) return GDX_OK;
   if (variant == 3 && !wslab_supported(p->K, p->NQ)) return GDX_ERR_UNSUPPORTED;
   int R[3];
+  if (variant == 2) {  // no tiles to build
+    batch_invalidate_problem(p->ctx, p);
+    lattice_shape(3, p->K, p->tileR);
+    p->kvariant3d = 2;
+    return GDX_OK;
+  }
+  if (!p->dev.W) {
+    const int old = p->kvariant3d;
+    p->kvariant3d = variant;
+    const int rc = points_alloc(p);
+    if (rc) {
+      p->kvariant3d = old;
+      return rc;
+    }
+  }
   if (variant >= 1) {
     tile3d_shape(p->K, R);
   } else {
@@ -443,7 +479,7 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
                   (p->D == 3 && p->desc.op_kind == GDX_OP_DIFFUSION && (p->kvariant3d == 0 || p->kvariant3d == 2)) ||
                   (p->desc.op_kind == GDX_OP_FLUX && gdx::flux_mixed_supported(p)),
               GDX_ERR_UNSUPPORTED,
-              "the FP32 form runs with the 3D z-marching or direct-store kernel (gdx_problem_set_kernel(prob, 0|2, rows)) "
+              "the FP32 form runs with the 3D pair-lattice or z-marching kernel (gdx_problem_set_kernel(prob, 0|2, rows)) "
               "or the fused 3D flux kernel (Q1, at most 2 Gauss points per direction)");
   if (precision != p->precision) gdx::batch_invalidate_problem(p->ctx, p);  // captured kernels change
   p->precision = precision;
@@ -512,7 +548,7 @@ int gdx_problem_set_kernel(gdx_problem *p, int32_t variant, int32_t rows_z) {
   variant &= ~GDX_KERNEL_HBM_PATTERNS;
   GDX_REQUIRE(p->symbolic_done && p->ctx, GDX_ERR_STATE, "needs gdx_symbolic and a device context");
   GDX_REQUIRE(variant >= 0 && variant <= 3, GDX_ERR_ARG,
-              "variant must be 0 (z-marching), 1 (per tile), 2 (per tile, direct stores) or 3 (per tile, wave slabs)");
+              "variant must be 0 (z-marching), 1 (per tile), 2 (pair lattice) or 3 (per tile, wave slabs)");
   GDX_REQUIRE(variant != 3 || gdx::wslab_supported(p->K, p->NQ), GDX_ERR_UNSUPPORTED,
               "the wave-slab kernel is built for Q2");
   GDX_REQUIRE(p->desc.op_kind == GDX_OP_DIFFUSION, GDX_ERR_UNSUPPORTED, "kernel variants are for the diffusion operator");

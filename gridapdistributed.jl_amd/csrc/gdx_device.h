@@ -117,36 +117,6 @@ __device__ __forceinline__ double uD_at(const KParams &kp, int g0, int g1, int g
   return kp.dir_coef[0] + kp.dir_coef[1] * x + kp.dir_coef[2] * y + kp.dir_coef[3] * z;
 }
 
-// Write one staged row from LDS to HBM in CSR order (contiguous stores) and,
-// for rows next to the Dirichlet boundary, subtract the lifting sum A_ij uD_j.
-template <int K, int DIM, int S>
-__device__ __forceinline__ void write_row(const double *__restrict__ row, long long rowstart, long long bidx, int pid,
-                                          int lenf, const int (&inv)[(S + 63) / 64], int g0, int g1, int g2,
-                                          const uint8_t *__restrict__ pat_fwd, double *__restrict__ values,
-                                          double *__restrict__ b, const KParams &kp) {
-  constexpr int W = 2 * K + 1;
-  const int lane = threadIdx.x & 63, len = lenf & 0xFFFF;
-  double *dst = values + rowstart;
-#pragma unroll
-  for (int kk = 0; kk < (S + 63) / 64; ++kk) {
-    const int k = lane + 64 * kk;
-    if (k < len) dst[k] = row[inv[kk]];
-  }
-  if (lenf >> 16) {
-    const uint8_t *fwd = pat_fwd + (size_t)pid * pattern_stride(S);
-    double acc = 0.0;
-    for (int sl = lane; sl < S; sl += 64) {
-      if (fwd[sl] == kSlotDirichlet) {
-        const int s1 = sl % W - K, s2 = (sl / W) % W - K, s3 = DIM == 3 ? sl / (W * W) - K : 0;
-        acc += row[sl] * uD_at(kp, g0 + s1, g1 + s2, g2 + s3);
-      }
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) b[bidx] -= acc;
-  }
-}
-
-
 // row table entry staged in LDS
 struct RowT {
   long long rowstart;

@@ -167,8 +167,8 @@ struct gdx_problem {
   std::vector<gdx::Tile> tiles;
   std::vector<int> tile_pats;
   int n_fast_tiles = 0;  // leading tiles whose position patterns fit in LDS
-  int kvariant3d = 0;    // 3D matrix kernel: 0 z-marching columns, 1 per-tile, 2 per-tile direct-store,
-                         // 3 per-tile wave-slab (Q2); chosen by the autotuner
+  int kvariant3d = 2;    // 3D matrix kernel: 0 z-marching columns, 1 per-tile, 2 pair lattice (the default),
+                         // 3 per-tile wave-slab (Q2)
   bool hbm_patterns = false;  // every tile takes the HBM-pattern kernel instance (GDX_KERNEL_HBM_PATTERNS)
   int precision = 0;     // contraction precision of the current numeric phase (GDX_PREC_*)
   int tileR[3] = {1, 1, 1};
@@ -194,6 +194,7 @@ struct gdx_problem {
   bool mapped = false;    // diffusion on a mapped grid (vertex coordinates in mapped_data)
   double diff_w = 1.0, reac_w = 0.0;  // mapped grids: diff_w kappa grad(u).grad(v) + reac_w u v
   void *mapped_data = nullptr;  // gdx_mapped.hip
+  void *lattice = nullptr;      // tables of the pair-lattice kernel (gdx_lattice.hip)
   void *pv = nullptr;     // PRange maps of the device PVectors (gdx_pvector.hip)
   std::vector<gdx_pvector *> pvecs;  // live PVectors on this problem
 };
@@ -273,8 +274,13 @@ int pattern_capacity_3d(int K, int NQ);
 int pattern_capacity_tile3d(int K, int NQ);
 void tile3d_shape(int K, int R[3]);
 int launch_matrix_tile3d(gdx_problem *p, hipStream_t st);
-int pattern_capacity_tile3d_direct(int K, int NQ);
-int launch_matrix_tile3d_direct(gdx_problem *p, hipStream_t st);
+// pair-lattice kernel (gdx_lattice.hip): 2D, and variant 2 in 3D
+int lattice_setup(gdx_problem *p);  // after the symbolic phase
+void lattice_free(gdx_problem *p);
+void lattice_shape(int dim, int K, int R[3]);  // rows per tile
+int launch_lattice(gdx_problem *p, hipStream_t st);
+bool lattice_used(const gdx_problem *p);  // the kernel of the problem's numeric phase on the uniform box
+int points_alloc(gdx_problem *p);  // kappa and f at the quadrature points, where the kernel reads them (gdx_capi.hip)
 bool wslab_supported(int K, int NQ);
 int pattern_capacity_tile3d_wslab(int K, int NQ);
 int launch_matrix_tile3d_wslab(gdx_problem *p, hipStream_t st);

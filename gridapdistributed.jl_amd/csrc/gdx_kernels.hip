@@ -125,177 +125,11 @@ __global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__
 }
 
 // ---------------------------------------------------------------------------
-// RHS f-part, sum-factorised: b_i = sum_q f(x_q) prod_d m_d(q; i_d),
-// m_d(q; i) = w_q h_d phi_a(q) over the cells containing node i.
-// ---------------------------------------------------------------------------
-template <int DIM, int K, int NQ, int R1, int R2, int R3>
-struct RhsTile {
-  static constexpr int C1 = R1 / K + 1, C2 = R2 / K + 1, C3 = DIM == 3 ? R3 / K + 1 : 1;
-  static constexpr int Q1 = C1 * NQ, Q2 = C2 * NQ, Q3 = DIM == 3 ? C3 * NQ : 1;
-  static constexpr int LF = Q1 * Q2 * Q3, LZ1 = R1 * Q3 * Q2, LZ2 = R1 * R2 * Q3;
-  static constexpr int NT = 256;
-};
-
-
-template <int DIM, int K, int NQ, int R1, int R2, int R3>
-__global__ __launch_bounds__(256) void k_rhs(const Tile *__restrict__ tiles, int ntiles,
-                                             const RowInfo *__restrict__ rowinfo, const double *__restrict__ F,
-                                             KParams kp, double *__restrict__ b) {
-  using T = RhsTile<DIM, K, NQ, R1, R2, R3>;
-  __shared__ double Fl[T::LF], Z1[T::LZ1], Z2[T::LZ2];
-  const int ti = tile_of_block(ntiles);
-  if (ti >= ntiles) return;
-  const Tile t = tiles[ti];
-  const int tid = threadIdx.x;
-  const int qs0 = (t.org[0] / K - 1) * NQ, qs1 = (t.org[1] / K - 1) * NQ;
-  const int qs2 = DIM == 3 ? (t.org[2] / K - 1) * NQ : 0;
-  for (int i = tid; i < T::LF; i += T::NT) {
-    const int a = i % T::Q1, c = (i / T::Q1) % T::Q2, e = i / (T::Q1 * T::Q2);
-    const int q0 = qs0 + a, q1 = qs1 + c, q2 = qs2 + e;
-    double v = 0.0;
-    if (q0 >= 0 && q0 < kp.qn[0] && q1 >= 0 && q1 < kp.qn[1] && q2 >= 0 && q2 < kp.qn[2])
-      v = F[q0 + (size_t)kp.qn[0] * (q1 + (size_t)kp.qn[1] * q2)];
-    Fl[i] = v;
-  }
-  __syncthreads();
-  // x: Z1[u1][q3][q2]
-  for (int i = tid; i < T::LZ1; i += T::NT) {
-    const int u1 = i / (T::Q3 * T::Q2), r = i % (T::Q3 * T::Q2);
-    const double *fr = Fl + r * T::Q1;
-    const int v = u1 + K, cmin = (v + K - 1) / K - 1, cmax = v / K;
-    double acc = 0.0;
-    for (int lc = cmin; lc <= cmax; ++lc)
-      for (int tt = 0; tt < NQ; ++tt) acc = fma(fr[lc * NQ + tt], node_factor<K, NQ>(kp, 0, u1, lc * NQ + tt), acc);
-    Z1[i] = acc;
-  }
-  __syncthreads();
-  // y: Z2[u1][u2][q3]
-  for (int i = tid; i < T::LZ2; i += T::NT) {
-    const int u1 = i / (R2 * T::Q3), u2 = (i / T::Q3) % R2, q3 = i % T::Q3;
-    const double *zr = Z1 + (u1 * T::Q3 + q3) * T::Q2;
-    const int v = u2 + K, cmin = (v + K - 1) / K - 1, cmax = v / K;
-    double acc = 0.0;
-    for (int lc = cmin; lc <= cmax; ++lc)
-      for (int tt = 0; tt < NQ; ++tt) acc = fma(zr[lc * NQ + tt], node_factor<K, NQ>(kp, 1, u2, lc * NQ + tt), acc);
-    Z2[i] = acc;
-  }
-  __syncthreads();
-  // z and store
-  for (int i = tid; i < R1 * R2 * (DIM == 3 ? R3 : 1); i += T::NT) {
-    const int u1 = i % R1, u2 = (i / R1) % R2, u3 = i / (R1 * R2);
-    if (u1 >= t.ext[0] || u2 >= t.ext[1] || u3 >= t.ext[2]) continue;
-    const RowInfo ri = rowinfo[t.rowinfo_base + row_index(t, t.org[0] + u1, t.org[1] + u2, t.org[2] + u3)];
-    if (ri.pid < 0) continue;
-    const double *zr = Z2 + (u1 * R2 + u2) * T::Q3;
-    double acc;
-    if (DIM == 3) {
-      const int v = u3 + K, cmin = (v + K - 1) / K - 1, cmax = v / K;
-      acc = 0.0;
-      for (int lc = cmin; lc <= cmax; ++lc)
-        for (int tt = 0; tt < NQ; ++tt) acc = fma(zr[lc * NQ + tt], node_factor<K, NQ>(kp, 2, u3, lc * NQ + tt), acc);
-    } else {
-      acc = zr[0];
-    }
-    b[ri.bidx] = acc;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 2D matrix kernel: one workgroup = one tile of R1 x R2 owned rows.
-// ---------------------------------------------------------------------------
-template <int K, int NQ, int R1, int R2>
-struct Tile2 {
-  static constexpr int C1 = R1 / K + 1, C2 = R2 / K + 1;
-  static constexpr int Q1 = C1 * NQ, Q2 = C2 * NQ;
-  static constexpr int NP1 = pair_count<K>(R1), NP2 = pair_count<K>(R2);
-  static constexpr int XS = Q2 | 1;
-  static constexpr int NT = 256;
-  static constexpr int W = 2 * K + 1, S = W * W;
-  static constexpr int LDS_KAPPA = Q1 * Q2, LDS_X = 2 * NP1 * XS, LDS_SLAB = R1 * R2 * S;
-  static constexpr int LDS_DOUBLES = LDS_KAPPA + LDS_X + LDS_SLAB;
-};
-
-template <int K, int NQ, int R1, int R2>
-__global__ __launch_bounds__(256) void k_assemble2d(const Tile *__restrict__ tiles, int ntiles,
-                                                    const RowInfo *__restrict__ rowinfo,
-                                                    const double *__restrict__ Wq, const uint8_t *__restrict__ pat_fwd,
-                                                    const uint8_t *__restrict__ pat_inv, double *__restrict__ values,
-                                                    double *__restrict__ b, KParams kp) {
-  using T = Tile2<K, NQ, R1, R2>;
-  constexpr int NINV = (T::S + 63) / 64;
-  __shared__ double lds[T::LDS_DOUBLES];
-  double *kap = lds;
-  double *XG = lds + T::LDS_KAPPA;
-  double *XM = XG + T::NP1 * T::XS;
-  double *slab = XM + T::NP1 * T::XS;
-  const int ti = tile_of_block(ntiles);
-  if (ti >= ntiles) return;
-  const Tile t = tiles[ti];
-  const int tid = threadIdx.x;
-  const int qs0 = (t.org[0] / K - 1) * NQ, qs1 = (t.org[1] / K - 1) * NQ;
-  for (int i = tid; i < T::LDS_KAPPA; i += T::NT) {
-    const int a = i % T::Q1, c = i / T::Q1;
-    const int q0 = qs0 + a, q1 = qs1 + c;
-    double v = 0.0;
-    if (q0 >= 0 && q0 < kp.qn[0] && q1 >= 0 && q1 < kp.qn[1]) v = Wq[q0 + (size_t)kp.qn[0] * q1];
-    kap[i] = v;
-  }
-  __syncthreads();
-  for (int it = tid; it < T::NP1 * T::Q2; it += T::NT) {
-    const int p1 = it / T::Q2, q2 = it % T::Q2;
-    int u, s, lc0, nc, a0, b0;
-    pair_natural<K>(p1, u, s);
-    pair_cells<K>(u, s, lc0, nc, a0, b0);
-    double xg = 0.0, xm = 0.0;
-    for (int tt = 0; tt < nc * NQ; ++tt) {
-      double G, M;
-      pair_factors<K, NQ>(kp, 0, a0, b0, tt, G, M);
-      const double k = kap[q2 * T::Q1 + lc0 * NQ + tt];
-      xg = fma(k, G, xg);
-      xm = fma(k, M, xm);
-    }
-    XG[p1 * T::XS + q2] = xg;
-    XM[p1 * T::XS + q2] = xm;
-  }
-  __syncthreads();
-  for (int it = tid; it < T::NP1 * T::NP2; it += T::NT) {
-    const int p1 = it % T::NP1, p2 = it / T::NP1;
-    int u1, s1, u2, s2, lc0, nc, a0, b0;
-    pair_natural<K>(p1, u1, s1);
-    pair_natural<K>(p2, u2, s2);
-    pair_cells<K>(u2, s2, lc0, nc, a0, b0);
-    double v = 0.0;
-    for (int tt = 0; tt < nc * NQ; ++tt) {
-      double G, M;
-      pair_factors<K, NQ>(kp, 1, a0, b0, tt, G, M);
-      v = fma(XG[p1 * T::XS + lc0 * NQ + tt], M, fma(XM[p1 * T::XS + lc0 * NQ + tt], G, v));
-    }
-    slab[(u2 * R1 + u1) * T::S + (s2 + K) * T::W + (s1 + K)] = v;
-  }
-  __syncthreads();
-  const int wave = tid >> 6, lane = tid & 63;
-  for (int rr = wave; rr < R1 * R2; rr += T::NT / 64) {
-    const int u1 = rr % R1, u2 = rr / R1;
-    if (u1 >= t.ext[0] || u2 >= t.ext[1]) continue;
-    const RowInfo ri = rowinfo[t.rowinfo_base + row_index(t, t.org[0] + u1, t.org[1] + u2, t.org[2])];
-    if (ri.pid < 0) continue;
-    int inv[NINV];
-#pragma unroll
-    for (int kk = 0; kk < NINV; ++kk) {
-      const int k = lane + 64 * kk;
-      inv[kk] = k < (ri.lenf & 0xFFFF) ? (int)pat_inv[(size_t)ri.pid * pattern_stride(T::S) + k] : 0;
-    }
-    write_row<K, 2, T::S>(slab + rr * T::S, ri.rowstart, ri.bidx, ri.pid, ri.lenf, inv, t.org[0] + u1,
-                          t.org[1] + u2, 0, pat_fwd, values, b, kp);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // launchers.  Tile shapes here must match tile_shape() in gdx_symbolic.cpp.
 // ---------------------------------------------------------------------------
-static unsigned grid_for(int ntiles) { return 8u * (unsigned)((ntiles + 7) / 8); }
-
 int launch_coefficients(gdx_problem *p, hipStream_t st) {
+  // the pair-lattice kernel takes a coefficient that is constant on every cell as it is
+  if (lattice_used(p) && (p->coef_cell || p->kp.nmodes == 0)) return GDX_OK;
   if (p->coef_cell) return launch_cell_coefficients(p, st);
   const KParams &kp = p->kp;
   int qnmax = kp.qn[0];
@@ -310,63 +144,29 @@ int launch_coefficients(gdx_problem *p, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-template <int DIM, int K, int NQ, int R1, int R2, int R3>
-static void rhs_run(gdx_problem *p, hipStream_t st) {
-  const int nt = (int)p->tiles.size();
-  hipLaunchKernelGGL((k_rhs<DIM, K, NQ, R1, R2, R3>), dim3(grid_for(nt)), dim3(256), 0, st, p->dev.tiles, nt,
-                     p->dev.rowinfo, p->dev.F, p->kp, p->dev.b);
-}
-
 int launch_matrix3d(gdx_problem *p, hipStream_t st, int precision);
-
-template <int K, int NQ, int R1, int R2>
-static void run2(gdx_problem *p, hipStream_t st) {
-  const int nt = (int)p->tiles.size();
-  hipLaunchKernelGGL((k_assemble2d<K, NQ, R1, R2>), dim3(grid_for(nt)), dim3(256), 0, st, p->dev.tiles, nt,
-                     p->dev.rowinfo, p->dev.W, p->dev.pat_fwd, p->dev.pat_inv, p->dev.values, p->dev.b, p->kp);
-}
 
 bool matrix_kernel_supported(int dim, int K, int NQ) {
   if (dim == 3) return (K == 2 && (NQ == 2 || NQ == 3)) || (K == 1 && NQ == 2);
   return dim == 2 && (K == 1 || K == 2) && (NQ == 2 || NQ == 3);
 }
 
+int launch_source(gdx_problem *p, hipStream_t st);
+
 int launch_rhs(gdx_problem *p, hipStream_t st) {
-  if (p->tiles.empty()) return GDX_OK;
-  const int K = p->K, NQ = p->NQ;
-  if (p->D == 3) {
-    if (p->kvariant3d != 1) return GDX_OK;  // the z-marching and direct-store kernels write b themselves
-    if (K == 2 && NQ == 3) rhs_run<3, 2, 3, 4, 8, 8>(p, st);
-    else if (K == 2 && NQ == 2) rhs_run<3, 2, 2, 4, 8, 8>(p, st);
-    else if (K == 1 && NQ == 2) rhs_run<3, 1, 2, 8, 8, 2>(p, st);
-    else return GDX_ERR_UNSUPPORTED;
-  } else {
-    if (K == 2 && NQ == 3) rhs_run<2, 2, 3, 16, 16, 1>(p, st);
-    else if (K == 2 && NQ == 2) rhs_run<2, 2, 2, 16, 16, 1>(p, st);
-    else if (K == 1 && NQ == 2) rhs_run<2, 1, 2, 16, 16, 1>(p, st);
-    else if (K == 1 && NQ == 3) rhs_run<2, 1, 3, 16, 16, 1>(p, st);
-    else return GDX_ERR_UNSUPPORTED;
-  }
-  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+  // the pair-lattice kernel takes a constant f in closed form, and the other
+  // kernels but the per-tile one write b themselves
+  const bool varies = p->kp.rhs_kind == GDX_RHS_MANUFACTURED && p->kp.nmodes > 0 && !p->coef_cell;
+  if (lattice_used(p) ? varies : p->kvariant3d == 1) return launch_source(p, st);
+  return GDX_OK;
 }
 
 int launch_matrix(gdx_problem *p, hipStream_t st) {
+  if (lattice_used(p)) return launch_lattice(p, st);  // either precision: its contractions are FP64
   if (p->tiles.empty()) return GDX_OK;
-  const int K = p->K, NQ = p->NQ;
-  if (p->D == 3) {
-    // the FP32 form exists for the z-marching and the direct-store kernels
-    if (p->precision == GDX_PREC_FP32 && p->kvariant3d == 0) return launch_matrix3d(p, st, GDX_PREC_FP32);
-    if (p->kvariant3d == 2) return launch_matrix_tile3d_direct(p, st);
-    if (p->kvariant3d == 3) return launch_matrix_tile3d_wslab(p, st);
-    return p->kvariant3d == 1 ? launch_matrix_tile3d(p, st) : launch_matrix3d(p, st, GDX_PREC_FP64);
-  } else {
-    if (K == 2 && NQ == 3) run2<2, 3, 16, 16>(p, st);
-    else if (K == 2 && NQ == 2) run2<2, 2, 16, 16>(p, st);
-    else if (K == 1 && NQ == 2) run2<1, 2, 16, 16>(p, st);
-    else if (K == 1 && NQ == 3) run2<1, 3, 16, 16>(p, st);
-    else return GDX_ERR_UNSUPPORTED;
-  }
-  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+  if (p->kvariant3d == 0) return launch_matrix3d(p, st, p->precision);
+  if (p->kvariant3d == 3) return launch_matrix_tile3d_wslab(p, st);
+  return launch_matrix_tile3d(p, st);
 }
 
 }  // namespace gdx

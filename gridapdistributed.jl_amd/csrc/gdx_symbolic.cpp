@@ -436,6 +436,31 @@ void tile_shape(int dim, int K, int R[3]) {
   }
 }
 
+void tile3d_shape(int K, int R[3]) {
+  R[0] = K == 2 ? 4 : 8;
+  R[1] = 8;
+  R[2] = K == 2 ? 8 : 2;
+}
+
+// tile shape of the problem's kernel; false where it takes none (the pair-lattice
+// kernel cuts its own tiles on the global lattice)
+static bool problem_tile_shape(const gdx_problem *p, int R[3]) {
+  tile_shape(p->D, p->K, R);
+  if (p->desc.op_kind == GDX_OP_FLUX) {
+    if (p->D == 3) R[1] = kFluxR2, R[2] = kFluxR3;
+    return true;
+  }
+  if (p->desc.op_kind != GDX_OP_DIFFUSION) return true;
+  if (p->D == 2 || p->kvariant3d == 2) return false;
+  if (p->kvariant3d != 0) tile3d_shape(p->K, R);
+  return true;
+}
+
+static void no_tiles(gdx_problem *p) {
+  p->tiles.clear();
+  p->tile_pats.clear();
+}
+
 // Host numbering, owners, global ids and row/col PRanges of every part.
 static void host_fe_stage(gdx_problem *p, const Ctx &c) {
   const int nparts = p->nparts;
@@ -784,9 +809,8 @@ static int host_csr_stage(gdx_problem *p, const Ctx &c) {
 
   // tiles of owned rows (the flux operator's fused kernel takes its own shape)
   int R[3];
-  tile_shape(c.D, K, R);
-  if (p->desc.op_kind == GDX_OP_FLUX && c.D == 3) R[1] = kFluxR2, R[2] = kFluxR3;
-  build_tiles(p, R);
+  if (problem_tile_shape(p, R)) build_tiles(p, R);
+  else no_tiles(p);
   return GDX_OK;
 }
 
@@ -863,8 +887,10 @@ int symbolic(gdx_problem *p) {
     if (rc != kUseHost) {
       if (rc) return rc;
       int R[3];
-      tile_shape(c.D, c.K, R);
-      if (p->desc.op_kind == GDX_OP_FLUX && c.D == 3) R[1] = kFluxR2, R[2] = kFluxR3;
+      if (!problem_tile_shape(p, R)) {
+        no_tiles(p);
+        return GDX_OK;
+      }
       const int rt = build_tiles_device(p, R);
       symbolic_mark("tiles (device)");
       return rt;

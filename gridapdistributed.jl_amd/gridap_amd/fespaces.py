@@ -321,7 +321,7 @@ class GpuProblem:
 
     def set_kernel(self, variant, rows_z=32):
         """3D matrix kernel: 0 z-marching columns (rows_z z rows per workgroup), 1 per tile,
-        2 per tile with direct stores, 3 per tile with wave-owned rows (Q2)."""
+        2 pair lattice (the default), 3 per tile with wave-owned rows (Q2)."""
         _lib.call("gdx_problem_set_kernel", self.handle, int(variant), int(rows_z))
 
     def get_kernel(self):

@@ -46,7 +46,8 @@ extern "C" {
 
 /* numeric precision of the cell contractions; the CSR values are FP64 */
 #define GDX_PREC_FP64 0
-#define GDX_PREC_FP32 1 /* mixed form: sum-factorised contractions in FP32 (3D, z-marching or direct-store kernel);
+#define GDX_PREC_FP32 1 /* mixed form, at least FP32 contractions: FP32 in the 3D z-marching kernel, FP64 in the
+                           3D pair-lattice kernel (where FP32 would gain nothing);
                            for GDX_OP_FLUX the cell Jacobians in FP32 (fused 3D Q1 kernel), residual FP64 */
 
 /* operator kinds */
@@ -152,10 +153,9 @@ int gdx_symbolic(gdx_problem *prob);
 int gdx_numeric(gdx_problem *prob, int32_t precision);
 
 /* 3D matrix kernel of a problem: variant 0 = z-marching columns with rows_z z
-   rows per workgroup (default 32), 1 = per-tile kernel, 2 = per-tile kernel
-   storing straight from registers, 3 = per-tile kernel whose waves own whole
-   rows (Q2 only; rows_z ignored for 1-3).  All give the same matrix to
-   rounding; gdx_batch_autotune picks the fastest. */
+   rows per workgroup, 1 = per-tile kernel, 2 = pair-lattice kernel (the
+   default), 3 = per-tile kernel whose waves own whole rows (Q2 only; rows_z
+   ignored for 1-3).  All give the same matrix to rounding. */
 int gdx_problem_set_kernel(gdx_problem *prob, int32_t variant, int32_t rows_z);
 /* variant flag: every tile reads its position patterns from HBM, as the tiles
    with more distinct patterns than the kernel's LDS holds always do (same
@@ -354,12 +354,10 @@ int gdx_fpcg(gdx_problem *prob, gdx_nn *nn, const double *rhs, double rtol, int3
 
 /* Batched numeric assembly: independent problems of uneven sizes and
    partitions (each after gdx_symbolic, all on one context) assembled by one
-   hipGraph launch.  gdx_batch_autotune times each 3D problem's matrix kernels
-   (z-marching columns of 16, 32 and 64 z rows per workgroup, the per-tile
-   kernel and its direct-store form) and keeps the fastest (chosen, per
-   problem, may be NULL: the z rows per workgroup, -1 for the per-tile kernel,
-   -2 for the direct-store form, -3 for the wave-slab form); the matrices
-   agree to rounding for every choice.  gdx_batch_capture records the numeric launches of every problem
+   hipGraph launch.  gdx_batch_autotune sets each 3D problem's matrix kernel to
+   the fastest form (chosen, per problem, may be NULL: minus the variant of
+   gdx_problem_set_kernel), which is the pair-lattice kernel at every measured
+   size, so nothing is timed.  gdx_batch_capture records the numeric launches of every problem
    (no memsets) as independent branches of one graph: the problems are spread over four streams
    (largest first, to the least loaded), forked from and joined back into the context's stream, so
    small problems run beside each other; gdx_batch_launch replays the graph on the context's stream
