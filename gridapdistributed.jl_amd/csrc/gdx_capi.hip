@@ -17,6 +17,8 @@ namespace gdx {
 int launch_coefficients(gdx_problem *p, hipStream_t st);
 int launch_rhs(gdx_problem *p, hipStream_t st);
 int launch_matrix(gdx_problem *p, hipStream_t st);
+bool points_used(const gdx_problem *p);  // the numeric phase fills kappa (and f) at the quadrature points
+bool source_used(const gdx_problem *p);  // and has a source-integral launch
 bool matrix_kernel_supported(int dim, int K, int NQ);
 
 static thread_local std::string g_last_error;
@@ -485,61 +487,61 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
   p->precision = precision;
   GDX_HIP(hipSetDevice(p->ctx->device));
   hipStream_t st = p->ctx->stream;
-  GDX_HIP(hipEventRecord(p->ev[0], st));
-  if (p->desc.op_kind == GDX_OP_FLUX) {
-    // residual_and_jacobian at the stored state: no coefficient or separate RHS phase
-    GDX_HIP(hipEventRecord(p->ev[1], st));
-    GDX_HIP(hipEventRecord(p->ev[2], st));
-    int rcf = gdx::flux_assemble(p, nullptr, false, precision == GDX_PREC_FP32, st);
-    if (rcf) {
-      set_error("flux operator launch failed");
-      return rcf;
+  for (bool &e : p->ev_set) e = false;
+  const bool diffusion = p->desc.op_kind == GDX_OP_DIFFUSION;
+  if (p->desc.op_kind == GDX_OP_FLUX || (diffusion && !p->mapped && !gdx::lattice_used(p))) {
+    // stages of several kernels: event records between them
+    GDX_HIP(hipEventRecord(p->ev[0], st));
+    if (!diffusion) {  // residual_and_jacobian at the stored state: no coefficient or separate RHS phase
+      if (int rc = gdx::flux_assemble(p, nullptr, false, precision == GDX_PREC_FP32, st)) {
+        set_error("flux operator launch failed");
+        return rc;
+      }
+    } else {
+      int rc = gdx::launch_coefficients(p, st);
+      if (!rc) {
+        GDX_HIP(hipEventRecord(p->ev[1], st));
+        rc = gdx::launch_rhs(p, st);
+      }
+      if (!rc) {
+        GDX_HIP(hipEventRecord(p->ev[2], st));
+        rc = gdx::launch_matrix(p, st);
+      }
+      if (rc) {
+        set_error("coefficient, rhs or matrix kernel launch failed");
+        return rc;
+      }
+      p->ev_set[1] = p->ev_set[2] = true;
     }
     GDX_HIP(hipEventRecord(p->ev[3], st));
+    p->ev_set[0] = p->ev_set[3] = true;
     return GDX_OK;
   }
-  if (p->desc.op_kind == GDX_OP_ELASTICITY) {
-    // matrix and RHS in one launch; no coefficient phase
-    GDX_HIP(hipEventRecord(p->ev[1], st));
-    GDX_HIP(hipEventRecord(p->ev[2], st));
-    int rce = gdx::elast_assemble(p, st);
-    if (rce) {
-      set_error("elasticity kernel launch failed");
-      return rce;
-    }
-    GDX_HIP(hipEventRecord(p->ev[3], st));
-    return GDX_OK;
+  // every other stage is timed by its own kernels' packets
+  int rc = GDX_OK;
+  auto stage = [&](bool used, int ends, auto &&launch) {
+    if (rc || !used) return;
+    p->launch_ev[0] = p->ev_set[0] ? nullptr : p->ev[0];
+    p->launch_ev[1] = p->ev[ends];
+    rc = launch();
+    p->launch_ev[0] = p->launch_ev[1] = nullptr;
+    p->ev_set[0] = p->ev_set[ends] = true;
+  };
+  if (!diffusion) {  // elasticity: matrix and RHS in one launch
+    stage(p->rows_total > 0, 3, [&] { return gdx::elast_assemble(p, st); });
+  } else if (p->mapped) {  // cell records (geometry, coefficients, cell matrices), then the rows
+    stage(true, 1, [&] { return gdx::mapped_assemble(p, st, 0); });
+    stage(gdx::mapped_rows(p) > 0, 3, [&] { return gdx::mapped_assemble(p, st, 1); });
+  } else {
+    stage(gdx::points_used(p), 1, [&] { return gdx::launch_coefficients(p, st); });
+    stage(gdx::source_used(p), 2, [&] { return gdx::launch_rhs(p, st); });
+    stage(true, 3, [&] { return gdx::launch_matrix(p, st); });
   }
-  if (p->mapped) {
-    // cell records (geometry, coefficients, cell matrices), then the rows
-    int rcm = gdx::mapped_assemble(p, st, 0);
-    GDX_HIP(hipEventRecord(p->ev[1], st));
-    GDX_HIP(hipEventRecord(p->ev[2], st));
-    if (!rcm) rcm = gdx::mapped_assemble(p, st, 1);
-    if (rcm) {
-      set_error("mapped-grid kernel launch failed");
-      return rcm;
-    }
-    GDX_HIP(hipEventRecord(p->ev[3], st));
-    return GDX_OK;
-  }
-  int rc = gdx::launch_coefficients(p, st);
   if (rc) {
-    set_error("coefficient kernel launch failed");
-    return rc;
+    for (bool &e : p->ev_set) e = false;
+    set_error("numeric kernel launch failed");
   }
-  GDX_HIP(hipEventRecord(p->ev[1], st));
-  if ((rc = gdx::launch_rhs(p, st))) {
-    set_error("rhs kernel launch failed");
-    return rc;
-  }
-  GDX_HIP(hipEventRecord(p->ev[2], st));
-  if ((rc = gdx::launch_matrix(p, st))) {
-    set_error("matrix kernel launch failed");
-    return rc;
-  }
-  GDX_HIP(hipEventRecord(p->ev[3], st));
-  return GDX_OK;
+  return rc;
 }
 
 int gdx_problem_set_kernel(gdx_problem *p, int32_t variant, int32_t rows_z) {
@@ -753,12 +755,15 @@ int gdx_phase_times(gdx_problem *p, double *ms, int32_t n) {
   GDX_REQUIRE(p && ms && n >= 0, GDX_ERR_ARG, "NULL argument");
   GDX_REQUIRE(p->symbolic_done, GDX_ERR_STATE, "gdx_symbolic has not run");
   GDX_REQUIRE(p->ctx, GDX_ERR_STATE, "host-only problem (created without a context)");
-  GDX_HIP(hipEventSynchronize(p->ev[3]));
   float t[4] = {0, 0, 0, 0};
-  GDX_HIP(hipEventElapsedTime(&t[0], p->ev[0], p->ev[1]));
-  GDX_HIP(hipEventElapsedTime(&t[1], p->ev[1], p->ev[2]));
-  GDX_HIP(hipEventElapsedTime(&t[2], p->ev[2], p->ev[3]));
-  GDX_HIP(hipEventElapsedTime(&t[3], p->ev[0], p->ev[3]));
+  int last = 0;
+  for (int k = 1; k < 4; ++k) {
+    if (!p->ev_set[k]) continue;
+    GDX_HIP(hipEventSynchronize(p->ev[k]));
+    GDX_HIP(hipEventElapsedTime(&t[k - 1], p->ev[last], p->ev[k]));
+    last = k;
+  }
+  if (last) GDX_HIP(hipEventElapsedTime(&t[3], p->ev[0], p->ev[last]));
   for (int i = 0; i < n && i < 4; ++i) ms[i] = t[i];
   return GDX_OK;
 }

@@ -500,7 +500,7 @@ int elast_assemble(gdx_problem *p, hipStream_t st) {
     const double *coef = p->coef_cell ? p->dev.cellk : p->dev.cell_lame;
     if (!coef) return GDX_ERR_STATE;
 #define GDX_ELAST_CW(KK, CW)                                                                                       \
-  hipLaunchKernelGGL((k_elast_cw<KK, kNodesPerWave, CW>), grid, block, 0, st, A, E->rows, E->sfac, E->sinfo, coef, \
+  GDX_LAUNCH(p, (k_elast_cw<KK, kNodesPerWave, CW>), grid, block, st, A, E->rows, E->sfac, E->sinfo, coef, \
                      E->mass, E->pinv, p->dev.values, p->dev.b)
     if (p->K == 2 && p->coef_cell) GDX_ELAST_CW(2, 1);
     else if (p->K == 2) GDX_ELAST_CW(2, 2);
@@ -510,10 +510,10 @@ int elast_assemble(gdx_problem *p, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
   }
   if (p->K == 2)
-    hipLaunchKernelGGL((k_elast<2, kNodesPerWave>), grid, block, 0, st, A, E->rows, E->fac, E->mass, E->pinv,
+    GDX_LAUNCH(p, (k_elast<2, kNodesPerWave>), grid, block, st, A, E->rows, E->fac, E->mass, E->pinv,
                        p->dev.values, p->dev.b);
   else
-    hipLaunchKernelGGL((k_elast<1, kNodesPerWave>), grid, block, 0, st, A, E->rows, E->fac, E->mass, E->pinv,
+    GDX_LAUNCH(p, (k_elast<1, kNodesPerWave>), grid, block, st, A, E->rows, E->fac, E->mass, E->pinv,
                        p->dev.values, p->dev.b);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }

@@ -1,5 +1,6 @@
 // Internal data structures of libgdx (host side).
 #pragma once
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -183,7 +184,12 @@ struct gdx_problem {
   gdx::DevNumbering dn;
   gdx::KParams kp{};
   gdx::Device dev;
+  // timing of the last numeric phase: start of its first kernel, ends of the
+  // coefficient, RHS and matrix stages (ev_set: the stages that launched)
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  bool ev_set[4] = {false, false, false, false};
+  // start and stop event of the next GDX_LAUNCH, nullptr outside gdx_numeric
+  hipEvent_t launch_ev[2] = {nullptr, nullptr};
   double phase_ms[4] = {0, 0, 0, 0};
   void *solve = nullptr;  // solver state (gdx_solve.hip), built on the first solve
   void *flux = nullptr;   // nonlinear operator state (gdx_flux.hip)
@@ -198,6 +204,17 @@ struct gdx_problem {
   void *pv = nullptr;     // PRange maps of the device PVectors (gdx_pvector.hip)
   std::vector<gdx_pvector *> pvecs;  // live PVectors on this problem
 };
+
+// Launch of a numeric phase's kernel.  The phase's events ride on the kernels'
+// own packets: an event record of its own costs a barrier and a cache flush,
+// about 5 us of the stream each.
+#define GDX_LAUNCH(p, kernel, grid, block, st, ...)                                                              \
+  do {                                                                                                           \
+    if ((p)->launch_ev[0] || (p)->launch_ev[1])                                                                  \
+      hipExtLaunchKernelGGL(kernel, grid, block, 0, st, (p)->launch_ev[0], (p)->launch_ev[1], 0, __VA_ARGS__);   \
+    else                                                                                                         \
+      hipLaunchKernelGGL(kernel, grid, block, 0, st, __VA_ARGS__);                                               \
+  } while (0)
 
 namespace gdx {
 void set_error(const std::string &msg);
@@ -308,6 +325,7 @@ void elast_free(gdx_problem *p);
 int elast_assemble(gdx_problem *p, hipStream_t st);
 int mapped_set(gdx_problem *p, const double *xyz);  // vertex coordinates; cell records and row list
 void mapped_free(gdx_problem *p);
+long long mapped_rows(const gdx_problem *p);  // owned free rows
 int mapped_assemble(gdx_problem *p, hipStream_t st, int stage);  // stage 0: cell records, 1: rows
 int flux_setup(gdx_problem *p);
 void flux_free(gdx_problem *p);

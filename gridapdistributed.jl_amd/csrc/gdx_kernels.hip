@@ -127,20 +127,26 @@ __global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__
 // ---------------------------------------------------------------------------
 // launchers.  Tile shapes here must match tile_shape() in gdx_symbolic.cpp.
 // ---------------------------------------------------------------------------
+bool points_used(const gdx_problem *p) { return !lattice_used(p) || (!p->coef_cell && p->kp.nmodes > 0); }
+
 int launch_coefficients(gdx_problem *p, hipStream_t st) {
   // the pair-lattice kernel takes a coefficient that is constant on every cell as it is
-  if (lattice_used(p) && (p->coef_cell || p->kp.nmodes == 0)) return GDX_OK;
+  if (!points_used(p)) return GDX_OK;
   if (p->coef_cell) return launch_cell_coefficients(p, st);
   const KParams &kp = p->kp;
   int qnmax = kp.qn[0];
   for (int d = 1; d < 3; ++d) qnmax = qnmax > kp.qn[d] ? qnmax : kp.qn[d];
   if (kp.nmodes > 0) {
     dim3 g1((qnmax + 255) / 256, kp.nmodes, 3);
-    hipLaunchKernelGGL(k_fourier_tables, g1, dim3(256), 0, st, p->dev.modes, kp, qnmax, p->dev.E);
+    const hipEvent_t stop = p->launch_ev[1];
+    p->launch_ev[1] = nullptr;
+    GDX_LAUNCH(p, k_fourier_tables, g1, dim3(256), st, p->dev.modes, kp, qnmax, p->dev.E);
+    p->launch_ev[0] = nullptr;
+    p->launch_ev[1] = stop;
   }
   const int bx = kp.qn[0] < 256 ? 64 * ((kp.qn[0] + 63) / 64) : 256;
   dim3 g2((kp.qn[0] + bx - 1) / bx, (kp.qn[1] + kCoefLines - 1) / kCoefLines, kp.qn[2]);
-  hipLaunchKernelGGL(k_coefficients, g2, dim3(bx), 0, st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, p->dev.F);
+  GDX_LAUNCH(p, k_coefficients, g2, dim3(bx), st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, p->dev.F);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
@@ -153,13 +159,14 @@ bool matrix_kernel_supported(int dim, int K, int NQ) {
 
 int launch_source(gdx_problem *p, hipStream_t st);
 
-int launch_rhs(gdx_problem *p, hipStream_t st) {
-  // the pair-lattice kernel takes a constant f in closed form, and the other
-  // kernels but the per-tile one write b themselves
-  const bool varies = p->kp.rhs_kind == GDX_RHS_MANUFACTURED && p->kp.nmodes > 0 && !p->coef_cell;
-  if (lattice_used(p) ? varies : p->kvariant3d == 1) return launch_source(p, st);
-  return GDX_OK;
+// the pair-lattice kernel takes a constant f in closed form, and the other
+// kernels but the per-tile one write b themselves
+bool source_used(const gdx_problem *p) {
+  const bool varies = p->ngdofs > 0 && p->kp.rhs_kind == GDX_RHS_MANUFACTURED && p->kp.nmodes > 0 && !p->coef_cell;
+  return lattice_used(p) ? varies : p->kvariant3d == 1;
 }
+
+int launch_rhs(gdx_problem *p, hipStream_t st) { return source_used(p) ? launch_source(p, st) : GDX_OK; }
 
 int launch_matrix(gdx_problem *p, hipStream_t st) {
   if (lattice_used(p)) return launch_lattice(p, st);  // either precision: its contractions are FP64

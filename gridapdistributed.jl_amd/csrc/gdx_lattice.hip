@@ -531,11 +531,11 @@ __global__ __launch_bounds__(256) void k_source(const LatArgs a, const double *_
 }
 
 template <int D, int K, int NQ>
-void launch_source(const LatArgs &a, const double *F, hipStream_t st) {
+void launch_source(gdx_problem *p, const LatArgs &a, const double *F, hipStream_t st) {
   constexpr int R[3] = {16, D == 3 ? 8 : 16, D == 3 ? 4 : 1};
   dim3 g((a.hi[0] - a.lo[0] + R[0] - 1) / R[0], (a.hi[1] - a.lo[1] + R[1] - 1) / R[1],
          (a.hi[2] - a.lo[2] + R[2] - 1) / R[2]);
-  if (g.x && g.y && g.z) hipLaunchKernelGGL((k_source<D, K, NQ>), g, dim3(256), 0, st, a, F);
+  if (g.x && g.y && g.z) GDX_LAUNCH(p, (k_source<D, K, NQ>), g, dim3(256), st, a, F);
 }
 
 template <int D, int K, int NQ>
@@ -646,7 +646,7 @@ int launch(gdx_problem *p, LatArgs &a, hipStream_t st) {
   for (int d = 0; d < 3; ++d) a.nt[d] = std::max(1, (a.hi[d] - a.lo[d] + R[d] - 1) / R[d]);
   const int64_t n = (int64_t)a.nt[0] * a.nt[1] * a.nt[2], lines = n / a.nt[0];
   const int64_t grid = 8 * ((lines + 7) / 8) * a.nt[0];
-  hipLaunchKernelGGL((k_lattice<T>), dim3((unsigned)grid), dim3(T::NT), 0, st, a, (int)n);
+  GDX_LAUNCH(p, (k_lattice<T>), dim3((unsigned)grid), dim3(T::NT), st, a, (int)n);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
@@ -785,13 +785,13 @@ int launch_source(gdx_problem *p, hipStream_t st) {
   fill_args(p, a, nqe);
   const double *F = p->dev.F;
   switch (p->D * 100 + p->K * 10 + p->NQ) {
-    case 323: launch_source<3, 2, 3>(a, F, st); break;
-    case 322: launch_source<3, 2, 2>(a, F, st); break;
-    case 312: launch_source<3, 1, 2>(a, F, st); break;
-    case 222: launch_source<2, 2, 2>(a, F, st); break;
-    case 223: launch_source<2, 2, 3>(a, F, st); break;
-    case 212: launch_source<2, 1, 2>(a, F, st); break;
-    case 213: launch_source<2, 1, 3>(a, F, st); break;
+    case 323: launch_source<3, 2, 3>(p, a, F, st); break;
+    case 322: launch_source<3, 2, 2>(p, a, F, st); break;
+    case 312: launch_source<3, 1, 2>(p, a, F, st); break;
+    case 222: launch_source<2, 2, 2>(p, a, F, st); break;
+    case 223: launch_source<2, 2, 3>(p, a, F, st); break;
+    case 212: launch_source<2, 1, 2>(p, a, F, st); break;
+    case 213: launch_source<2, 1, 3>(p, a, F, st); break;
     default: return GDX_ERR_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;

@@ -81,6 +81,11 @@ __global__ void k_pv_axpy(int64_t n, double a, const double *__restrict__ x, dou
   if (i < n) y[i] = fma(a, x[i], y[i]);
 }
 
+__global__ void k_pv_copy(int64_t n, const double *__restrict__ s, double *__restrict__ d) {
+  const int64_t i = blockIdx.x * (int64_t)kB + threadIdx.x;
+  if (i < n) d[i] = s[i];
+}
+
 __global__ void k_pv_fill(int64_t n, double a, double *__restrict__ y) {
   const int64_t i = blockIdx.x * (int64_t)kB + threadIdx.x;
   if (i < n) y[i] = a;
@@ -407,9 +412,9 @@ int gdx_pvector_copy_rhs(gdx_pvector *v) {
     return GDX_ERR_STATE;
   }
   hipStream_t st = v->p->ctx->stream;
-  if (v->n > 0 && hipMemcpyAsync(v->v, v->p->dev.b, v->n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess)
-    return GDX_ERR_HIP;
-  return GDX_OK;
+  // a kernel of ours queues behind the assembly's at once; a runtime copy waits for a barrier packet first
+  if (v->n > 0) hipLaunchKernelGGL(gdx::k_pv_copy, dim3(gdx::nblk(v->n)), dim3(gdx::kB), 0, st, v->n, v->p->dev.b, v->v);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
 int gdx_pvector_consistent(gdx_pvector *v) {
