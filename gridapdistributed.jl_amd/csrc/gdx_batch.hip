@@ -7,12 +7,13 @@
 //                       against 0.79 (z-marching) and 0.63 (per tile); Q1
 //                       131 x 97 x 75 0.050 ms against 0.45
 //   gdx_batch_capture   records every problem's numeric launches (coefficient,
-//                       RHS and matrix kernels; no memsets) into one hipGraph
-//                       of independent branches: the problems are spread over
-//                       kBranches streams (largest first, each to the branch
-//                       with the least work), forked from and joined back into
-//                       the context's stream, so small problems that fill few
-//                       CUs run beside each other and beside the large ones
+//                       RHS and matrix kernels; no memsets) into one hipGraph:
+//                       the diffusion problems on the uniform box go together,
+//                       the tiles of all of them in one launch (and their
+//                       coefficients in two); the others are independent
+//                       branches, spread over kBranches streams (largest first,
+//                       each to the branch with the least work), forked from
+//                       and joined back into the context's stream
 //   gdx_batch_launch    replays it on the context's stream
 //
 #include <hip/hip_runtime.h>
@@ -27,6 +28,9 @@ struct gdx_batch {
   std::vector<gdx_problem *> probs;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  // the diffusion problems on the uniform box, together in a few launches
+  gdx::LatticeBatch *lattice = nullptr;
+  gdx::CoefBatch *coef = nullptr;
   // capture-time fork/join streams and events (default priority)
   std::vector<hipStream_t> side;
   std::vector<hipEvent_t> ev;  // [0] fork, [1..] joins
@@ -69,6 +73,13 @@ void drop_graph(gdx_batch *b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;
+  if (b->lattice || b->coef) {  // a replay in flight reads the tables
+    if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
+    gdx::lattice_batch_free(b->lattice);
+    gdx::coef_batch_free(b->coef);
+    b->lattice = nullptr;
+    b->coef = nullptr;
+  }
 }
 
 }  // namespace
@@ -122,19 +133,37 @@ int gdx_batch_capture(gdx_batch *b) {
   drop_graph(b);
   if (hipStreamSynchronize(st) != hipSuccess) return fail(GDX_ERR_HIP, "stream failed");
   if (ensure_branches(b)) return fail(GDX_ERR_HIP, "stream or event creation failed");
-  // largest problems first, each to the least loaded branch (work = stored values);
-  // within a branch the problems keep the batch order
-  const int nb = std::min<int>(kBranches, (int)b->probs.size());
-  std::vector<size_t> order(b->probs.size());
+  // the diffusion problems of the pair-lattice kernel go together, on the first branch
+  std::vector<gdx_problem *> lat, points, rest;
+  double lat_work = 0.0;
+  for (gdx_problem *p : b->probs) {
+    if (p->desc.op_kind != GDX_OP_DIFFUSION || p->mapped || !gdx::lattice_used(p)) {
+      rest.push_back(p);
+      continue;
+    }
+    lat.push_back(p);
+    if (gdx::points_used(p)) points.push_back(p);
+    lat_work += (double)p->nnz_total;
+  }
+  if ((!lat.empty() && gdx::lattice_batch_build(lat, &b->lattice)) ||
+      (!points.empty() && gdx::coef_batch_build(points, &b->coef))) {
+    drop_graph(b);
+    return fail(GDX_ERR_ALLOC, "the batch's tables do not fit in device memory");
+  }
+  // the others: largest first, each to the least loaded branch (work = stored values);
+  // within a branch they keep the batch order
+  const int nb = std::max(1, std::min<int>(kBranches, (int)rest.size() + (lat.empty() ? 0 : 1)));
+  std::vector<size_t> order(rest.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(),
-                   [&](size_t x, size_t y) { return b->probs[x]->nnz_total > b->probs[y]->nnz_total; });
-  std::vector<int> branch(b->probs.size(), 0);
+                   [&](size_t x, size_t y) { return rest[x]->nnz_total > rest[y]->nnz_total; });
+  std::vector<int> branch(rest.size(), 0);
   std::vector<double> load(nb, 0.0);
+  load[0] = lat_work;
   for (size_t i : order) {
     const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     branch[i] = k;
-    load[k] += (double)b->probs[i]->nnz_total + 1.0;
+    load[k] += (double)rest[i]->nnz_total + 1.0;
   }
   auto stream_of = [&](int k) { return k == 0 ? st : b->side[k - 1]; };
   if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess)
@@ -143,7 +172,10 @@ int gdx_batch_capture(gdx_batch *b) {
   if (hipEventRecord(b->ev[0], st) != hipSuccess) rc = GDX_ERR_HIP;
   for (int k = 1; k < nb && !rc; ++k)
     if (hipStreamWaitEvent(stream_of(k), b->ev[0], 0) != hipSuccess) rc = GDX_ERR_HIP;
-  for (size_t i = 0; i < b->probs.size() && !rc; ++i) rc = gdx::numeric_launches(b->probs[i], stream_of(branch[i]));
+  if (!rc && b->coef) rc = gdx::coef_batch_launch(b->coef, st);
+  for (size_t i = 0; i < points.size() && !rc; ++i) rc = gdx::launch_rhs(points[i], st);
+  if (!rc && b->lattice) rc = gdx::lattice_batch_launch(b->lattice, st);
+  for (size_t i = 0; i < rest.size() && !rc; ++i) rc = gdx::numeric_launches(rest[i], stream_of(branch[i]));
   // join every side branch that was forked, also after a failed launch, so the capture can end
   for (int k = 1; k < nb; ++k)
     if (hipEventRecord(b->ev[k], stream_of(k)) != hipSuccess || hipStreamWaitEvent(st, b->ev[k], 0) != hipSuccess)
@@ -152,6 +184,7 @@ int gdx_batch_capture(gdx_batch *b) {
   const hipError_t e = hipStreamEndCapture(st, &g);
   if (rc || e != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
+    drop_graph(b);
     return fail(rc ? rc : GDX_ERR_HIP, "graph capture failed");
   }
   b->graph = g;

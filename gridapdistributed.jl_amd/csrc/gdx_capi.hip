@@ -15,10 +15,7 @@
 
 namespace gdx {
 int launch_coefficients(gdx_problem *p, hipStream_t st);
-int launch_rhs(gdx_problem *p, hipStream_t st);
 int launch_matrix(gdx_problem *p, hipStream_t st);
-bool points_used(const gdx_problem *p);  // the numeric phase fills kappa (and f) at the quadrature points
-bool source_used(const gdx_problem *p);  // and has a source-integral launch
 bool matrix_kernel_supported(int dim, int K, int NQ);
 
 static thread_local std::string g_last_error;

@@ -296,6 +296,19 @@ int lattice_setup(gdx_problem *p);  // after the symbolic phase
 void lattice_free(gdx_problem *p);
 void lattice_shape(int dim, int K, int R[3]);  // rows per tile
 int launch_lattice(gdx_problem *p, hipStream_t st);
+// many problems' coefficients and tiles in a few launches (their device tables
+// hold the problems' current buffers and coefficient modes)
+struct LatticeBatch;
+struct CoefBatch;
+int lattice_batch_build(const std::vector<gdx_problem *> &ps, LatticeBatch **out);
+int lattice_batch_launch(const LatticeBatch *b, hipStream_t st);
+void lattice_batch_free(LatticeBatch *b);
+int coef_batch_build(const std::vector<gdx_problem *> &ps, CoefBatch **out);  // problems with points_used
+int coef_batch_launch(const CoefBatch *b, hipStream_t st);
+void coef_batch_free(CoefBatch *b);
+bool points_used(const gdx_problem *p);  // the numeric phase fills kappa (and f) at the quadrature points
+bool source_used(const gdx_problem *p);  // and has a source-integral launch
+int launch_rhs(gdx_problem *p, hipStream_t st);
 bool lattice_used(const gdx_problem *p);  // the kernel of the problem's numeric phase on the uniform box
 int points_alloc(gdx_problem *p);  // kappa and f at the quadrature points, where the kernel reads them (gdx_capi.hip)
 bool wslab_supported(int K, int NQ);

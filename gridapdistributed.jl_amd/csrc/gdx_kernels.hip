@@ -22,6 +22,9 @@
 // neighbouring parts' contributions at the source, ghost rows stay zero.
 #include <hip/hip_runtime.h>
 
+#include <new>
+#include <vector>
+
 #include "gdx_device.h"
 
 namespace gdx {
@@ -31,10 +34,10 @@ namespace gdx {
 // a_m exp(i theta_m) = [a_m exp(i phi_m) exp(2 pi i k_m1 x)] exp(2 pi i k_m2 y) exp(2 pi i k_m3 z)
 // with the three 1D factors tabulated once per launch.
 // ---------------------------------------------------------------------------
-__global__ void k_fourier_tables(const double *__restrict__ modes, KParams kp, int qnmax, double *__restrict__ E) {
-  const int m = blockIdx.y, d = blockIdx.z;
+__device__ __forceinline__ void fourier_table(const double *__restrict__ modes, const KParams &kp, int qnmax,
+                                              double *__restrict__ E, int m, int d, int first, int step) {
   const double *M = modes + 5 * m;
-  for (int q = threadIdx.x + blockIdx.x * blockDim.x; q < qnmax; q += blockDim.x * gridDim.x) {
+  for (int q = first; q < qnmax; q += step) {
     double x = 0.0;
     if (d < kp.dim && q < kp.qn[d]) {
       const int c = q / kp.NQ, t = q % kp.NQ;
@@ -56,6 +59,11 @@ __global__ void k_fourier_tables(const double *__restrict__ modes, KParams kp, i
   }
 }
 
+__global__ void k_fourier_tables(const double *__restrict__ modes, KParams kp, int qnmax, double *__restrict__ E) {
+  fourier_table(modes, kp, qnmax, E, blockIdx.y, blockIdx.z, threadIdx.x + blockIdx.x * blockDim.x,
+                blockDim.x * gridDim.x);
+}
+
 // One block = LINES consecutive x-lines (q2 .. q2+LINES-1 at fixed q3) of the
 // quadrature lattice; thread <-> q1.  The x factors of a chunk of modes stay
 // in registers across the lines; the per-line (y,z) products b = e2 e3 and
@@ -63,12 +71,12 @@ __global__ void k_fourier_tables(const double *__restrict__ modes, KParams kp, i
 //   g += Re(e1 b),  s += Im(e1 (k.c) b).
 constexpr int kCoefLines = 8, kCoefModes = 16;
 
-__global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__ modes,
-                                                      const double *__restrict__ E, KParams kp, int qnmax,
-                                                      double *__restrict__ W, double *__restrict__ F) {
+__device__ __forceinline__ void coefficient_lines(const double *__restrict__ modes, const double *__restrict__ E,
+                                                  const KParams &kp, int qnmax, double *__restrict__ W,
+                                                  double *__restrict__ F, int bx, int by, int q3) {
   __shared__ double tb[kCoefLines][kCoefModes][4];  // br, bi, (k.c) br, (k.c) bi
-  const int q1 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int q2b = blockIdx.y * kCoefLines, q3 = blockIdx.z;
+  const int q1 = bx * blockDim.x + threadIdx.x;
+  const int q2b = by * kCoefLines;
   const bool active = q1 < kp.qn[0];
   const int nm = kp.nmodes;
   double g[kCoefLines], s[kCoefLines];
@@ -124,9 +132,49 @@ __global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__
   }
 }
 
+__global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__ modes,
+                                                      const double *__restrict__ E, KParams kp, int qnmax,
+                                                      double *__restrict__ W, double *__restrict__ F) {
+  coefficient_lines(modes, E, kp, qnmax, W, F, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// The same for many problems at once: a block finds its problem and its place
+// in that problem's grid in a table.
+struct CoefProblem {
+  KParams kp;
+  const double *modes;
+  double *E, *W, *F;
+  int qnmax;
+};
+// one wave per block: small problems' lines are 32..96 points, a larger block
+// would leave most of its lanes idle
+struct CoefBlock {
+  int prob, x, y, z;
+};
+
+__global__ __launch_bounds__(256) void k_fourier_tables_batch(const CoefProblem *__restrict__ probs,
+                                                              const CoefBlock *__restrict__ blocks) {
+  const CoefBlock b = blocks[blockIdx.x];
+  const CoefProblem &p = probs[b.prob];
+  fourier_table(p.modes, p.kp, p.qnmax, p.E, b.y, b.z, threadIdx.x, blockDim.x);
+}
+
+__global__ __launch_bounds__(64) void k_coefficients_batch(const CoefProblem *__restrict__ probs,
+                                                            const CoefBlock *__restrict__ blocks) {
+  const CoefBlock b = blocks[blockIdx.x];
+  const CoefProblem &p = probs[b.prob];
+  coefficient_lines(p.modes, p.E, p.kp, p.qnmax, p.W, p.F, b.x, b.y, b.z);
+}
+
 // ---------------------------------------------------------------------------
 // launchers.  Tile shapes here must match tile_shape() in gdx_symbolic.cpp.
 // ---------------------------------------------------------------------------
+static int longest_line(const KParams &kp) {
+  int qnmax = kp.qn[0];
+  for (int d = 1; d < 3; ++d) qnmax = qnmax > kp.qn[d] ? qnmax : kp.qn[d];
+  return qnmax;
+}
+
 bool points_used(const gdx_problem *p) { return !lattice_used(p) || (!p->coef_cell && p->kp.nmodes > 0); }
 
 int launch_coefficients(gdx_problem *p, hipStream_t st) {
@@ -134,8 +182,7 @@ int launch_coefficients(gdx_problem *p, hipStream_t st) {
   if (!points_used(p)) return GDX_OK;
   if (p->coef_cell) return launch_cell_coefficients(p, st);
   const KParams &kp = p->kp;
-  int qnmax = kp.qn[0];
-  for (int d = 1; d < 3; ++d) qnmax = qnmax > kp.qn[d] ? qnmax : kp.qn[d];
+  const int qnmax = longest_line(kp);
   if (kp.nmodes > 0) {
     dim3 g1((qnmax + 255) / 256, kp.nmodes, 3);
     const hipEvent_t stop = p->launch_ev[1];
@@ -147,6 +194,60 @@ int launch_coefficients(gdx_problem *p, hipStream_t st) {
   const int bx = kp.qn[0] < 256 ? 64 * ((kp.qn[0] + 63) / 64) : 256;
   dim3 g2((kp.qn[0] + bx - 1) / bx, (kp.qn[1] + kCoefLines - 1) / kCoefLines, kp.qn[2]);
   GDX_LAUNCH(p, k_coefficients, g2, dim3(bx), st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, p->dev.F);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+// Coefficients of many problems in two launches.  Alone each problem's pair of
+// launches fills a few CUs and ends in a gap: 32 Q1 cubes of 16..48 cells took
+// 32 x (4 + 10) us of kernels.
+struct CoefBatch {
+  CoefProblem *probs = nullptr;
+  CoefBlock *tables = nullptr, *lines = nullptr;
+  unsigned ntables = 0, nlines = 0;
+};
+
+void coef_batch_free(CoefBatch *b) {
+  if (!b) return;
+  void *ptrs[] = {b->probs, b->tables, b->lines};
+  for (void *q : ptrs)
+    if (q) (void)hipFree(q);
+  delete b;
+}
+
+int coef_batch_build(const std::vector<gdx_problem *> &ps, CoefBatch **out) {
+  *out = nullptr;
+  std::vector<CoefProblem> probs;
+  std::vector<CoefBlock> tables, lines;
+  for (gdx_problem *p : ps) {
+    const KParams &kp = p->kp;
+    const int i = (int)probs.size();
+    probs.push_back({kp, p->dev.modes, p->dev.E, p->dev.W, p->dev.F, longest_line(kp)});
+    for (int d = 0; d < 3; ++d)
+      for (int m = 0; m < kp.nmodes; ++m) tables.push_back({i, 0, m, d});
+    for (int z = 0; z < kp.qn[2]; ++z)
+      for (int y = 0; y < (kp.qn[1] + kCoefLines - 1) / kCoefLines; ++y)
+        for (int x = 0; x < (kp.qn[0] + 63) / 64; ++x) lines.push_back({i, x, y, z});
+  }
+  CoefBatch *b = new (std::nothrow) CoefBatch;
+  if (!b) return GDX_ERR_ALLOC;
+  auto put = [](auto **dst, const auto &src) {
+    const size_t n = src.size() * sizeof(src[0]);
+    return hipMalloc(reinterpret_cast<void **>(dst), n ? n : 1) == hipSuccess &&
+           (!n || hipMemcpy(*dst, src.data(), n, hipMemcpyHostToDevice) == hipSuccess);
+  };
+  if (!put(&b->probs, probs) || !put(&b->tables, tables) || !put(&b->lines, lines)) {
+    coef_batch_free(b);
+    return GDX_ERR_ALLOC;
+  }
+  b->ntables = (unsigned)tables.size();
+  b->nlines = (unsigned)lines.size();
+  *out = b;
+  return GDX_OK;
+}
+
+int coef_batch_launch(const CoefBatch *b, hipStream_t st) {
+  if (b->ntables) hipLaunchKernelGGL(k_fourier_tables_batch, dim3(b->ntables), dim3(256), 0, st, b->probs, b->tables);
+  if (b->nlines) hipLaunchKernelGGL(k_coefficients_batch, dim3(b->nlines), dim3(64), 0, st, b->probs, b->lines);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 

@@ -419,21 +419,39 @@ __device__ __forceinline__ void lattice_tile(ArgsRef a, int tile) {
     lines(l0, l1 < H ? l1 : H, std::integral_constant<int, 2>{});
     lines(l0 > H ? l0 : H, l1, std::integral_constant<int, 1>{});
   } else {
-    constexpr int RPI = 64 / T::L;  // rows per iteration of the wave
+    // 64 / L rows per wave instruction, four instructions at a time: their row
+    // entries, then their values, then the stores
+    constexpr int RPI = 64 / T::L, G = 4, STEP = T::NW * RPI;
     const int sub = lane / T::L, k = lane % T::L;
     int cur = -1, dl = 0;
-#pragma unroll 2
-    for (int r = wave * RPI + sub; r < (T::ROWS + RPI - 1) / RPI * RPI; r += T::NW * RPI) {
-      LatRowL e{0, 0, 0};
-      if (r < T::ROWS) e = rows[r];
-      const int len = e.meta & 0xFF;
-      if (__any(len != 0 && e.meta != cur)) {
-        if (len) {
-          dl = (int16_t)a.delta[(size_t)(e.meta >> 9) * T::PSTR + k];
-          cur = e.meta;
-        }
+#pragma unroll 1
+    for (int r0 = wave * RPI; r0 < T::ROWS; r0 += G * STEP) {
+      LatRowL e[G];
+      bool other = false;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const int r = r0 + g * STEP + sub;
+        e[g] = rows[r < T::ROWS ? r : 0];
+        if (r >= T::ROWS) e[g].meta = 0;
+        other = other || ((e[g].meta & 0xFF) && e[g].meta != cur);
       }
-      if (k < len) *reinterpret_cast<double *>(reinterpret_cast<char *>(a.values) + e.off + 8 * k) = U[e.ub + dl];
+      int d[G];
+      if (__any(other)) {  // another position pattern: its offsets, one wait for the four rows
+#pragma unroll
+        for (int g = 0; g < G; ++g) d[g] = (int16_t)a.delta[(size_t)(e[g].meta >> 9) * T::PSTR + k];
+        cur = e[G - 1].meta;
+        dl = d[G - 1];
+      } else {
+#pragma unroll
+        for (int g = 0; g < G; ++g) d[g] = dl;
+      }
+      double v[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) v[g] = U[e[g].ub + d[g]];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (k < (e[g].meta & 0xFF))
+          *reinterpret_cast<double *>(reinterpret_cast<char *>(a.values) + e[g].off + 8 * k) = v[g];
     }
   }
   // b: one lane per row
@@ -464,6 +482,18 @@ __global__ __launch_bounds__(T::NT, T::WPS) void k_lattice(const LatArgs, int nt
   const int nx = args->nt[0], i = (int)(blockIdx.x / 8), line = (i / nx) * 8 + (int)((blockIdx.x + i / nx) % 8);
   const int tile = line * nx + i % nx;
   if (tile < ntiles) lattice_tile<T>(*args, tile);
+}
+
+// The tiles of many problems in one launch: a block finds its problem and tile
+// in a table.
+struct LatBlock {
+  int prob, tile;
+};
+template <class T>
+__global__ __launch_bounds__(T::NT, T::WPS) void k_lattice_batch(const LatArgs *probs, const LatBlock *blocks) {
+  typedef const __attribute__((address_space(4))) LatBlock *BlockPtr;
+  const int prob = ((BlockPtr)blocks)[blockIdx.x].prob, tile = ((BlockPtr)blocks)[blockIdx.x].tile;
+  lattice_tile<T>(((ArgsPtr)probs)[prob], tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -641,13 +671,43 @@ void geometry(const gdx_problem *p, LatArgs &a) {
 }
 
 template <class T>
-int launch(gdx_problem *p, LatArgs &a, hipStream_t st) {
+int64_t cut_tiles(LatArgs &a) {
   const int R[3] = {T::R1, T::R2, T::R3};
   for (int d = 0; d < 3; ++d) a.nt[d] = std::max(1, (a.hi[d] - a.lo[d] + R[d] - 1) / R[d]);
-  const int64_t n = (int64_t)a.nt[0] * a.nt[1] * a.nt[2], lines = n / a.nt[0];
+  return (int64_t)a.nt[0] * a.nt[1] * a.nt[2];
+}
+
+template <class T>
+int launch(gdx_problem *p, LatArgs &a, hipStream_t st) {
+  const int64_t n = cut_tiles<T>(a), lines = n / a.nt[0];
   const int64_t grid = 8 * ((lines + 7) / 8) * a.nt[0];
   GDX_LAUNCH(p, (k_lattice<T>), dim3((unsigned)grid), dim3(T::NT), st, a, (int)n);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+template <class T>
+int launch_batch(const LatArgs *probs, const LatBlock *blocks, unsigned n, hipStream_t st) {
+  hipLaunchKernelGGL((k_lattice_batch<T>), dim3(n), dim3(T::NT), 0, st, probs, blocks);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+// the instance of (dim, order, points per cell and direction) `key`
+template <class F>
+int with_shape(int key, F &&f) {
+  switch (key) {
+    case 321: return f(ShapeOf<3, 2, 1>::type{});
+    case 322: return f(ShapeOf<3, 2, 2>::type{});
+    case 323: return f(ShapeOf<3, 2, 3>::type{});
+    case 311: return f(ShapeOf<3, 1, 1>::type{});
+    case 312: return f(ShapeOf<3, 1, 2>::type{});
+    case 221: return f(ShapeOf<2, 2, 1>::type{});
+    case 222: return f(ShapeOf<2, 2, 2>::type{});
+    case 223: return f(ShapeOf<2, 2, 3>::type{});
+    case 211: return f(ShapeOf<2, 1, 1>::type{});
+    case 212: return f(ShapeOf<2, 1, 2>::type{});
+    case 213: return f(ShapeOf<2, 1, 3>::type{});
+  }
+  return GDX_ERR_UNSUPPORTED;
 }
 
 // arguments of the problem's numeric launch; nqe = points per cell and direction
@@ -802,21 +862,78 @@ int launch_lattice(gdx_problem *p, hipStream_t st) {
   LatArgs a{};
   int nqe = 1;
   fill_args(p, a, nqe);
-  const int key = p->D * 100 + p->K * 10 + nqe;
-  switch (key) {
-    case 321: return launch<ShapeOf<3, 2, 1>::type>(p, a, st);
-    case 322: return launch<ShapeOf<3, 2, 2>::type>(p, a, st);
-    case 323: return launch<ShapeOf<3, 2, 3>::type>(p, a, st);
-    case 311: return launch<ShapeOf<3, 1, 1>::type>(p, a, st);
-    case 312: return launch<ShapeOf<3, 1, 2>::type>(p, a, st);
-    case 221: return launch<ShapeOf<2, 2, 1>::type>(p, a, st);
-    case 222: return launch<ShapeOf<2, 2, 2>::type>(p, a, st);
-    case 223: return launch<ShapeOf<2, 2, 3>::type>(p, a, st);
-    case 211: return launch<ShapeOf<2, 1, 1>::type>(p, a, st);
-    case 212: return launch<ShapeOf<2, 1, 2>::type>(p, a, st);
-    case 213: return launch<ShapeOf<2, 1, 3>::type>(p, a, st);
+  return with_shape(p->D * 100 + p->K * 10 + nqe, [&](auto shape) { return launch<decltype(shape)>(p, a, st); });
+}
+
+// Tiles of many problems, one launch per instance.  A small problem's own launch
+// fills a few CUs: 32 Q1 cubes of 16..48 cells on four branches of a graph took
+// 0.65 ms, the single launch (with the coefficients' two) 0.2 ms.
+struct LatticeBatch {
+  LatArgs *probs = nullptr;
+  struct Group {
+    int key;
+    LatBlock *blocks;
+    unsigned n;
+  };
+  std::vector<Group> groups;
+};
+
+void lattice_batch_free(LatticeBatch *b) {
+  if (!b) return;
+  if (b->probs) (void)hipFree(b->probs);
+  for (LatticeBatch::Group &g : b->groups)
+    if (g.blocks) (void)hipFree(g.blocks);
+  delete b;
+}
+
+int lattice_batch_build(const std::vector<gdx_problem *> &ps, LatticeBatch **out) {
+  *out = nullptr;
+  std::vector<LatArgs> probs;
+  std::vector<int> keys;
+  std::vector<std::vector<LatBlock>> blocks;
+  for (gdx_problem *p : ps) {
+    if (!p->lattice) return GDX_ERR_STATE;
+    LatArgs a{};
+    int nqe = 1;
+    fill_args(p, a, nqe);
+    const int key = p->D * 100 + p->K * 10 + nqe;
+    int64_t n = 0;
+    const int rc = with_shape(key, [&](auto shape) {
+      n = cut_tiles<decltype(shape)>(a);
+      return GDX_OK;
+    });
+    if (rc) return rc;
+    const size_t g = std::find(keys.begin(), keys.end(), key) - keys.begin();
+    if (g == keys.size()) {
+      keys.push_back(key);
+      blocks.emplace_back();
+    }
+    for (int64_t t = 0; t < n; ++t) blocks[g].push_back({(int)probs.size(), (int)t});
+    probs.push_back(a);
   }
-  return GDX_ERR_UNSUPPORTED;
+  LatticeBatch *b = new (std::nothrow) LatticeBatch;
+  if (!b) return GDX_ERR_ALLOC;
+  bool ok = put(&b->probs, probs) == hipSuccess;
+  for (size_t g = 0; g < keys.size(); ++g) {
+    b->groups.push_back({keys[g], nullptr, (unsigned)blocks[g].size()});
+    ok = ok && put(&b->groups.back().blocks, blocks[g]) == hipSuccess;
+  }
+  if (!ok) {
+    lattice_batch_free(b);
+    return GDX_ERR_ALLOC;
+  }
+  *out = b;
+  return GDX_OK;
+}
+
+int lattice_batch_launch(const LatticeBatch *b, hipStream_t st) {
+  for (const LatticeBatch::Group &g : b->groups) {
+    const int rc = with_shape(g.key, [&](auto shape) {
+      return launch_batch<decltype(shape)>(b->probs, g.blocks, g.n, st);
+    });
+    if (rc) return rc;
+  }
+  return GDX_OK;
 }
 
 }  // namespace gdx
