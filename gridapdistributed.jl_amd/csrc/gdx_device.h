@@ -117,6 +117,30 @@ __device__ __forceinline__ double uD_at(const KParams &kp, int g0, int g1, int g
   return kp.dir_coef[0] + kp.dir_coef[1] * x + kp.dir_coef[2] * y + kp.dir_coef[3] * z;
 }
 
+// sum_k val[k] x[col[k]] of one row by LPR lanes: each lane's share, U entries at
+// a time with their values and ids loaded before the first gather (one at a time
+// every entry waited for its id, then for its x).  Values and ids are read once.
+template <int LPR, int U>
+__device__ __forceinline__ double row_product(const double *__restrict__ val, const int *__restrict__ col, int len,
+                                              int lane, const double *__restrict__ x) {
+  double acc = 0.0;
+  for (int k0 = lane; k0 < len; k0 += LPR * U) {
+    double v[U], xv[U];
+    int c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = k0 + u * LPR < len;
+      c[u] = in ? __builtin_nontemporal_load(col + k0 + u * LPR) : -1;
+      v[u] = in ? __builtin_nontemporal_load(val + k0 + u * LPR) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) xv[u] = c[u] >= 0 ? x[c[u]] : 0.0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = fma(v[u], xv[u], acc);
+  }
+  return acc;
+}
+
 // row table entry staged in LDS
 struct RowT {
   long long rowstart;

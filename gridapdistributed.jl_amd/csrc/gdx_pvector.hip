@@ -22,7 +22,7 @@
 #include <new>
 #include <vector>
 
-#include "gdx_internal.h"
+#include "gdx_device.h"
 
 struct gdx_pvector {
   gdx_problem *p = nullptr;  // nullptr once the problem released its device memory
@@ -109,8 +109,7 @@ __global__ __launch_bounds__(kB) void k_pv_mul(int64_t nrows, const long long *_
   double acc = 0.0;
   if (row < nrows) {
     const long long s = rstart[row], cb = rcb[row];
-    const int len = rlen[row];
-    for (int k = lane; k < len; k += LPR) acc = fma(val[s + k], x[cb + colidx[s + k]], acc);
+    acc = row_product<LPR, 4>(val + s, colidx + s, rlen[row], lane, x + cb);
   }
 #pragma unroll
   for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, LPR);
@@ -249,7 +248,9 @@ int build_mul(gdx_problem *p) {
     std::copy(P.colidx.begin(), P.colidx.end(), colidx.begin() + P.val_base);
     cbase += P.ncols;
   }
-  D->lpr = maxlen > 64 ? 32 : (maxlen > 32 ? 16 : 8);
+  // Q2 rows (27..125 entries, 62 on average): 16 lanes keep 94% of their loads in
+  // use, 32 lanes 80%
+  D->lpr = maxlen > 192 ? 32 : (maxlen > 32 ? 16 : 8);
   if (!upload(&D->rstart, rstart) || !upload(&D->rlen, rlen) || !upload(&D->rcb, rcb) ||
       !upload(&D->colidx, colidx)) {
     set_error("device allocation failed for the local CSR column ids");
