@@ -62,6 +62,7 @@ namespace gdx {
 void twogrid_free(gdx_nn *nn);
 int twogrid_attach(gdx_nn *nn, gdx_problem *p);
 int twogrid_apply(void *nn, const double *r, double *z, hipStream_t st);
+FpcgPrec twogrid_prec(gdx_nn *nn, bool current);  // current: attached to the matrix's present values
 int twogrid_train_step(gdx_nn *nn, uint64_t seed, float lr, int smooth_passes, float *loss);
 gdx_problem *twogrid_problem(gdx_nn *nn);
 void twogrid_options(gdx_nn *nn, int sweeps, bool use_net);

@@ -403,9 +403,10 @@ static void spmv(gdx_problem *p, SolveData *s, const double *x, double *y, hipSt
 }
 
 static void dot2(SolveData *s, const double *a, const double *b, const double *c, const double *d, double *out,
-                 hipStream_t st) {
-  const int nb = std::min(kRedBlocks, std::max(1, (s->n + kBlk - 1) / kBlk));
-  hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(kBlk), 0, st, s->n, a, b, c, d, s->part);
+                 hipStream_t st, int n = -1) {
+  if (n < 0) n = s->n;
+  const int nb = std::min(kRedBlocks, std::max(1, (n + kBlk - 1) / kBlk));
+  hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(kBlk), 0, st, n, a, b, c, d, s->part);
   hipLaunchKernelGGL(k_finish2, dim3(1), dim3(kBlk), 0, st, s->part, nb, out);
 }
 
@@ -606,8 +607,23 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
     hipLaunchKernelGGL(k_gather_b, g, b, 0, st, n, s->bidx, p->dev.b, s->b);
   }
   hipLaunchKernelGGL(k_inv_diag, g, b, 0, st, n, s->dpos, p->dev.values, s->dinv);
-  (void)hipMemsetAsync(s->x, 0, n * sizeof(double), st);
-  if (hipMemcpyAsync(s->r, s->b, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) return GDX_ERR_HIP;
+  // the iteration's vectors: global-id order, or the preconditioner's lattice
+  double *vx = s->x, *vr = s->r, *vz = s->z, *vp = s->p, *vq = s->q;
+  int nv = n;
+  if (prec->begin) {
+    double *v[5];
+    if ((rc = prec->begin(prec->ctx, s->b, prec->current, &nv, v, st))) return rc;
+    vx = v[0], vr = v[1], vz = v[2], vp = v[3], vq = v[4];
+  } else if (hipMemcpyAsync(vr, s->b, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
+    return GDX_ERR_HIP;
+  }
+  const dim3 gv((nv + kBlk - 1) / kBlk);
+  auto product = [&](const double *x, double *y) {
+    if (prec->begin) prec->product(prec->ctx, x, y, st);
+    else spmv(p, s, x, y, st);
+  };
+  const auto apply = prec->begin ? prec->apply_lattice : prec->apply;
+  (void)hipMemsetAsync(vx, 0, nv * sizeof(double), st);
   dot2(s, s->b, s->b, nullptr, nullptr, s->sc + 6, st);
   double bb;
   if (hipMemcpyAsync(&bb, s->sc + 6, sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -617,18 +633,18 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
   bool fall = false, nonfinite = false;
   double last_check = bnorm;
   if (bnorm > 0.0) {
-    if ((rc = prec->apply(prec->ctx, s->r, s->z, st))) return rc;
-    if (hipMemcpyAsync(s->p, s->z, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) return GDX_ERR_HIP;
+    if ((rc = apply(prec->ctx, vr, vz, st))) return rc;
+    if (hipMemcpyAsync(vp, vz, nv * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) return GDX_ERR_HIP;
     IterGraph G;
     for (it = 1; it <= maxiter; ++it) {
       rc = run_iteration(st, G, [&]() {
-        spmv(p, s, s->p, s->q, st);
-        dot2(s, s->p, s->q, s->p, s->r, s->sc, st);  // sc[0] = pq, sc[1] = pr
-        hipLaunchKernelGGL(k_fcg_update, g, b, 0, st, n, s->sc, s->x, s->r, s->p, s->q);
-        int r2 = prec->apply(prec->ctx, s->r, s->z, st);
+        product(vp, vq);
+        dot2(s, vp, vq, vp, vr, s->sc, st, nv);  // sc[0] = pq, sc[1] = pr
+        hipLaunchKernelGGL(k_fcg_update, gv, b, 0, st, nv, s->sc, vx, vr, vp, vq);
+        int r2 = apply(prec->ctx, vr, vz, st);
         if (r2) return r2;
-        dot2(s, s->z, s->q, s->r, s->r, s->sc + 2, st);  // sc[2] = zq, sc[3] = rr
-        hipLaunchKernelGGL(k_fcg_dir, g, b, 0, st, n, s->sc, s->z, s->p);
+        dot2(s, vz, vq, vr, vr, s->sc + 2, st, nv);  // sc[2] = zq, sc[3] = rr
+        hipLaunchKernelGGL(k_fcg_dir, gv, b, 0, st, nv, s->sc, vz, vp);
         return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
       });
       if (rc) return rc;
@@ -657,6 +673,7 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
     }
     if (it > maxiter) it = maxiter;
   }
+  if (prec->begin) prec->end(prec->ctx, vx, s->x, st);
   if (fall) {
     // Jacobi-PCG from the current iterate (or from zero if it is not finite);
     // s->b still holds the right-hand side
@@ -762,7 +779,6 @@ int solve_newton(gdx_problem *p, const gdx_newton_opts *o, double *xh, gdx_newto
   };
   // FPCG with the two-grid preconditioner, rebuilt from the current Jacobian
   // (fine diagonal and Galerkin coarse operator), or Jacobi-PCG
-  const FpcgPrec prec{twogrid_apply, o->precond};
   int fallbacks = 0;
   auto correct = [&](int *li) -> int {
     const auto ts = clk::now();
@@ -770,6 +786,7 @@ int solve_newton(gdx_problem *p, const gdx_newton_opts *o, double *xh, gdx_newto
     int r, fb = 0;
     if (o->precond) {
       if ((r = twogrid_attach(o->precond, p))) return r;
+      const FpcgPrec prec = twogrid_prec(o->precond, true);
       r = fpcg_run(p, s, &prec, nullptr, o->lin_rtol, o->lin_maxiter, li, &rr, &fb);
       fallbacks += fb;
     } else {

@@ -68,6 +68,8 @@ struct TwoGrid {
   double *ec = nullptr, *ec2 = nullptr;      // training: coarse error [n^3]
   float *tgt = nullptr;
   const double *dinv = nullptr;
+  int *asym = nullptr;     // 1: fst is not symmetric to the bit
+  double *lat = nullptr;   // lattice vectors of the flexible CG: x r z p q t1 t2 t3 dinv, nf^3 each
   double *fst = nullptr;   // fine matrix as a 27-point stencil on the lattice [27][nf^3]
   double *cst = nullptr;   // Galerkin coarse operator P^T A P as a stencil [27][n^3]
   double *rc = nullptr;    // coarse residual R s [n^3]
@@ -847,15 +849,80 @@ void rms(TwoGrid *T, const double *a, const float *fa, int64_t count, double *ds
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(kB), 0, st, T->red, kRed, (double)count, mode, dst);
 }
 
-// network input from a fine residual in global-id order (s into red[kS]);
-// with the network off only the coarse residual rc is formed
-void make_input(gdx_nn *nn, TwoGrid *T, const double *r, hipStream_t st, bool for_net = true) {
+// offset of the stencil's slot s on the lattice
+__device__ __forceinline__ int slot_offset(int s, int nf) {
+  return (s % 3 - 1) + nf * ((s / 3) % 3 - 1) + nf * nf * (s / 9 - 1);
+}
+
+// *asym = 1 if the stencil is not symmetric to the bit
+__global__ __launch_bounds__(kB) void k_asymmetric(int nf, const double *__restrict__ fst, int *__restrict__ asym) {
+  const int tot = nf * nf * nf, i = blockIdx.x * kB + threadIdx.x;
+  int bad = 0;
+  if (i < tot) {
+#pragma unroll
+    for (int s = 14; s < 27; ++s) {
+      const int j = i + slot_offset(s, nf);
+      const double u = fst[(size_t)s * tot + i], l = j < tot ? fst[(size_t)(26 - s) * tot + j] : 0.0;
+      bad |= __double_as_longlong(u) != __double_as_longlong(l);
+    }
+  }
+  if (__syncthreads_or(bad) && threadIdx.x == 0) *asym = 1;
+}
+
+// y = A x on the fine lattice (boundary nodes 0), or y = r - A x.  A is the
+// 27-plane stencil fst; where it is symmetric only its upper 14 planes are
+// read, the lower offsets' coefficients being the upper ones of the neighbour,
+// which the same XCD has read shortly before (each takes a contiguous run of
+// nodes).  The bound is the planes' bytes: 14 x 8 per node against 10 x 27 + 28
+// for the CSR product with 16-bit column codes, and no gather through ids.
+// 128^3 cells: 80 us (the CSR product 144); 96^3: 25 us, its planes staying in the
+// last-level cache (62).
+template <bool RESID>
+__global__ __launch_bounds__(kB) void k_lattice_product(int nf, const double *__restrict__ fst,
+                                                        const int *__restrict__ asym, const double *__restrict__ x,
+                                                        const double *__restrict__ r, double *__restrict__ y) {
+  const int tot = nf * nf * nf, nblk = (tot + kB - 1) / kB, per = (nblk + 7) / 8;
+  const int blk = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int i = blk * kB + threadIdx.x;
+  if (i >= tot) return;
+  const int a = i % nf, b = (i / nf) % nf, c = i / (nf * nf);
+  if (a == 0 || b == 0 || c == 0 || a == nf - 1 || b == nf - 1 || c == nf - 1) {
+    y[i] = 0.0;
+    return;
+  }
+  const bool sym = __builtin_amdgcn_readfirstlane(*asym) == 0;
+  double up[13], lo[13], xu[13], xl[13];
+#pragma unroll
+  for (int k = 0; k < 13; ++k) {
+    const int s = 14 + k, o = slot_offset(s, nf);
+    up[k] = fst[(size_t)s * tot + i];
+    lo[k] = (fst + (sym ? (int64_t)s * tot - o : (int64_t)(26 - s) * tot))[i];
+    xu[k] = x[i + o];
+    xl[k] = x[i - o];
+  }
+  double acc = fst[(size_t)13 * tot + i] * x[i];
+#pragma unroll
+  for (int k = 0; k < 13; ++k) acc = fma(up[k], xu[k], fma(lo[k], xl[k], acc));
+  y[i] = RESID ? r[i] - acc : acc;
+}
+
+void lattice_product(TwoGrid *T, const double *x, const double *r, double *y, hipStream_t st) {
+  const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
+  const dim3 g(8 * ((nb(nfl) + 7) / 8)), b(kB);
+  if (r) hipLaunchKernelGGL(k_lattice_product<true>, g, b, 0, st, T->nf, T->fst, T->asym, x, r, y);
+  else hipLaunchKernelGGL(k_lattice_product<false>, g, b, 0, st, T->nf, T->fst, T->asym, x, nullptr, y);
+}
+
+// network input from a fine residual in global-id order, or on the lattice (s
+// into red[kS]); with the network off only the coarse residual rc is formed
+void make_input(gdx_nn *nn, TwoGrid *T, const double *r, hipStream_t st, bool for_net = true, bool lattice = false) {
   nn::Net &N = nn->net;
   const int64_t v = (int64_t)T->n * T->n * T->n;
   // restriction reads only interior lattice nodes, all of which the scatter
   // writes: no clearing (and no memset, so this can be captured in a graph)
-  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, T->flat);
-  hipLaunchKernelGGL(k_restrict, dim3(nb(v)), dim3(kB), 0, st, T->n, T->nf, T->flat, T->dlat, T->rho, T->rc);
+  if (!lattice) hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, T->flat);
+  hipLaunchKernelGGL(k_restrict, dim3(nb(v)), dim3(kB), 0, st, T->n, T->nf, lattice ? r : T->flat, T->dlat, T->rho,
+                     T->rc);
   if (!for_net) return;
   rms(T, T->rho, nullptr, v, T->red + kS, 0, st);
   hipLaunchKernelGGL(k_input0, dim3(nb(v)), dim3(kB), 0, st, v, T->rho, T->red + kS, N.inp_f);
@@ -999,11 +1066,21 @@ void twogrid_free(gdx_nn *nn) {
   if (!T) return;
   mg_free(T);
   void *ptrs[] = {T->gid_node, T->flat, T->dlat, T->t1, T->t2, T->t3, T->rho, T->red, T->ec, T->ec2, T->tgt,
-                  T->fst, T->cst, T->rc, T->ca, T->cb};
+                  T->fst, T->cst, T->rc, T->ca, T->cb, T->lat};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   delete T;
   nn->tg = nullptr;
+}
+
+// the fine matrix's current values as a stencil on the lattice
+static int fine_stencil(TwoGrid *T, hipStream_t st) {
+  const long long *rs = nullptr;
+  const int *rl = nullptr, *cg = nullptr;
+  if (int rc = solve_csr_view(T->prob, &rs, &rl, &cg)) return rc;
+  hipLaunchKernelGGL(k_fine_stencil, dim3((unsigned)std::max(1, (T->ng + kFsRows - 1) / kFsRows)), dim3(kB), 0, st,
+                     T->ng, T->nf, rs, rl, cg, T->prob->dev.values, T->gid_node, T->fst);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
 // bind the network to a problem's current matrix: transfer maps, the fine
@@ -1063,6 +1140,8 @@ int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
       twogrid_free(nn);
       return GDX_ERR_ALLOC;
     }
+    // the entries of absent neighbours stay zero: one matrix pattern for as long as the attachment lasts
+    if (hipMemsetAsync(T->fst, 0, 27 * nfl * sizeof(double), st) != hipSuccess) return GDX_ERR_HIP;
     if (p->dev_numbering ? gid_node_device(p, T->gid_node) != GDX_OK
                          : hipMemcpy(T->gid_node, gid_node.data(), gid_node.size() * sizeof(long long),
                                      hipMemcpyHostToDevice) != hipSuccess)
@@ -1075,30 +1154,18 @@ int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
   hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, T->dinv, T->dlat);
   hipLaunchKernelGGL(k_input1, dim3(nb(v)), dim3(kB), 0, st, n, nf, p->kp.h[0], T->dlat, N.inp_f + v);
   // fine stencil and the Galerkin coarse operator of the current matrix
-  const long long *rs = nullptr;
-  const int *rl = nullptr, *cg = nullptr;
-  if ((rc = solve_csr_view(p, &rs, &rl, &cg))) return rc;
-  if (hipMemsetAsync(T->fst, 0, 27 * nfl * sizeof(double), st) != hipSuccess) return GDX_ERR_HIP;
-  hipLaunchKernelGGL(k_fine_stencil, dim3((unsigned)std::max(1, (T->ng + kFsRows - 1) / kFsRows)), dim3(kB), 0, st,
-                     T->ng, nf, rs, rl, cg, p->dev.values, T->gid_node, T->fst);
+  if ((rc = fine_stencil(T, st))) return rc;
   galerkin(n, nf, 0, nfl, T->fst, T->cst, st);
   if ((rc = mg_setup(T, st))) return rc;
   return hipStreamSynchronize(st) == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-// z = M r (device vectors in global-id order)
-int twogrid_apply(void *ctx, const double *r, double *z, hipStream_t st) {
-  gdx_nn *nn = reinterpret_cast<gdx_nn *>(ctx);
-  TwoGrid *T = tg_of(nn);
-  if (!T) return GDX_ERR_STATE;
+// the coarse correction of the fine residual s (global-id order, or on the
+// lattice): its prolongation in T->flat
+static int coarse_correction(gdx_nn *nn, TwoGrid *T, const double *s, bool lattice, double *flat, hipStream_t st) {
   nn::Net &N = nn->net;
-  gdx_problem *p = T->prob;
-  const int ng = T->ng;
   const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
-  hipLaunchKernelGGL(k_jacobi0, dim3(nb(ng)), dim3(kB), 0, st, ng, kOmega, T->dinv, r, z);
-  solve_spmv_dev(p, z, T->t1, st);
-  hipLaunchKernelGGL(k_rminus, dim3(nb(ng)), dim3(kB), 0, st, ng, r, T->t1);
-  make_input(nn, T, T->t1, st, T->use_net);
+  make_input(nn, T, s, st, T->use_net, lattice);
   if (T->use_net) {
     int rc = N.forward_dev();
     if (rc) return rc;
@@ -1126,14 +1193,101 @@ int twogrid_apply(void *ctx, const double *r, double *z, hipStream_t st) {
       std::swap(ea, eb);
     }
   }
-  hipLaunchKernelGGL(k_prolong_d, dim3(nb(nfl)), dim3(kB), 0, st, T->n, T->nf, ea, T->flat);
+  hipLaunchKernelGGL(k_prolong_d, dim3(nb(nfl)), dim3(kB), 0, st, T->n, T->nf, ea, flat);
+  return GDX_OK;
+}
+
+// z += alpha c + w D^-1 (s - alpha Ac), alpha the energy-optimal step along c
+static void coarse_step(TwoGrid *T, int n, const double *dinv, const double *s, const double *c, const double *ac,
+                        double *z, hipStream_t st) {
+  hipLaunchKernelGGL(k_dot2p, dim3(kRed), dim3(kB), 0, st, n, c, s, c, ac, T->red);
+  hipLaunchKernelGGL(k_alpha, dim3(1), dim3(kB), 0, st, T->red, T->red + kS + 5);
+  hipLaunchKernelGGL(k_coarse_post, dim3(nb(n)), dim3(kB), 0, st, n, kOmega, T->red + kS + 5, dinv, s, c, ac, z);
+}
+
+// z = M r (device vectors in global-id order)
+int twogrid_apply(void *ctx, const double *r, double *z, hipStream_t st) {
+  gdx_nn *nn = reinterpret_cast<gdx_nn *>(ctx);
+  TwoGrid *T = tg_of(nn);
+  if (!T) return GDX_ERR_STATE;
+  gdx_problem *p = T->prob;
+  const int ng = T->ng;
+  hipLaunchKernelGGL(k_jacobi0, dim3(nb(ng)), dim3(kB), 0, st, ng, kOmega, T->dinv, r, z);
+  solve_spmv_dev(p, z, T->t1, st);
+  hipLaunchKernelGGL(k_rminus, dim3(nb(ng)), dim3(kB), 0, st, ng, r, T->t1);
+  if (int rc = coarse_correction(nn, T, T->t1, false, T->flat, st)) return rc;
   hipLaunchKernelGGL(k_gather, dim3(nb(ng)), dim3(kB), 0, st, ng, T->gid_node, T->flat, T->t2);  // c
   solve_spmv_dev(p, T->t2, T->t3, st);                                                             // A c
-  hipLaunchKernelGGL(k_dot2p, dim3(kRed), dim3(kB), 0, st, ng, T->t2, T->t1, T->t2, T->t3, T->red);
-  hipLaunchKernelGGL(k_alpha, dim3(1), dim3(kB), 0, st, T->red, T->red + kS + 5);
-  hipLaunchKernelGGL(k_coarse_post, dim3(nb(ng)), dim3(kB), 0, st, ng, kOmega, T->red + kS + 5, T->dinv, T->t1,
-                     T->t2, T->t3, z);
+  coarse_step(T, ng, T->dinv, T->t1, T->t2, T->t3, z, st);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+// The flexible CG on the fine lattice: its vectors hold every lattice node
+// (boundary nodes zero), so neither the transfers nor the products permute.
+// lattice vectors in T->lat
+enum { kLx, kLr, kLz, kLp, kLq, kLt1, kLt2, kLt3, kLdinv, kLcount };
+
+static int lattice_begin(void *ctx, const double *r, bool current, int *n, double *vecs[5], hipStream_t st) {
+  TwoGrid *T = tg_of(reinterpret_cast<gdx_nn *>(ctx));
+  const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
+  if (!current)
+    if (int rc = fine_stencil(T, st)) return rc;
+  // boundary nodes zero: r's and D^-1's here, x's by the solver, and with them every other vector's
+  if (hipMemsetAsync(T->asym, 0, sizeof(int), st) != hipSuccess ||
+      hipMemsetAsync(T->lat + kLr * nfl, 0, nfl * sizeof(double), st) != hipSuccess ||
+      hipMemsetAsync(T->lat + kLdinv * nfl, 0, nfl * sizeof(double), st) != hipSuccess)
+    return GDX_ERR_HIP;
+  hipLaunchKernelGGL(k_asymmetric, dim3(nb(nfl)), dim3(kB), 0, st, T->nf, T->fst, T->asym);
+  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, T->dinv, T->lat + kLdinv * nfl);
+  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, T->lat + kLr * nfl);
+  for (int k = 0; k < 5; ++k) vecs[k] = T->lat + k * nfl;
+  *n = (int)nfl;
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+static void lattice_mul(void *ctx, const double *x, double *y, hipStream_t st) {
+  lattice_product(tg_of(reinterpret_cast<gdx_nn *>(ctx)), x, nullptr, y, st);
+}
+
+static int lattice_apply(void *ctx, const double *r, double *z, hipStream_t st) {
+  gdx_nn *nn = reinterpret_cast<gdx_nn *>(ctx);
+  TwoGrid *T = tg_of(nn);
+  const int nfl = T->nf * T->nf * T->nf;
+  double *t1 = T->lat + (size_t)kLt1 * nfl, *t2 = T->lat + (size_t)kLt2 * nfl, *t3 = T->lat + (size_t)kLt3 * nfl;
+  const double *dinv = T->lat + (size_t)kLdinv * nfl;
+  hipLaunchKernelGGL(k_jacobi0, dim3(nb(nfl)), dim3(kB), 0, st, nfl, kOmega, dinv, r, z);
+  lattice_product(T, z, r, t1, st);
+  if (int rc = coarse_correction(nn, T, t1, true, t2, st)) return rc;
+  lattice_product(T, t2, nullptr, t3, st);
+  coarse_step(T, nfl, dinv, t1, t2, t3, z, st);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+static void lattice_end(void *ctx, const double *xl, double *x, hipStream_t st) {
+  TwoGrid *T = tg_of(reinterpret_cast<gdx_nn *>(ctx));
+  hipLaunchKernelGGL(k_gather, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, xl, x);
+}
+
+FpcgPrec twogrid_prec(gdx_nn *nn, bool current) {
+  FpcgPrec p{};
+  p.apply = twogrid_apply;
+  p.ctx = nn;
+  TwoGrid *T = tg_of(nn);
+  const int64_t nfl = T ? (int64_t)T->nf * T->nf * T->nf : 0;
+  if (!T || nfl >= (int64_t)1 << 30) return p;  // 32-bit node ids in the kernels
+  if (!T->lat && hipMalloc(reinterpret_cast<void **>(&T->lat), (kLcount * nfl + 1) * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
+    T->lat = nullptr;  // no room: the products from the CSR rows, in global-id order
+  }
+  if (T->lat) {
+    T->asym = reinterpret_cast<int *>(T->lat + kLcount * nfl);
+    p.begin = lattice_begin;
+    p.product = lattice_mul;
+    p.apply_lattice = lattice_apply;
+    p.end = lattice_end;
+    p.current = current;
+  }
+  return p;
 }
 
 // one training step on a fresh sample; loss (relative squared error) to *loss
@@ -1384,7 +1538,7 @@ int gdx_fpcg(gdx_problem *prob, gdx_nn *nn, const double *rhs, double rtol, int3
     return GDX_ERR_STATE;
   }
   if (hipSetDevice(prob->ctx->device) != hipSuccess) return GDX_ERR_HIP;
-  gdx::FpcgPrec pr{gdx::twogrid_apply, nn};
+  const gdx::FpcgPrec pr = nn ? gdx::twogrid_prec(nn, false) : gdx::FpcgPrec{};
   int it = 0, fb = 0;
   int rc = gdx::solve_fpcg(prob, nn ? &pr : nullptr, rhs, rtol, maxiter, xsol, &it, relres, ms, &fb);
   if (iters) *iters = it;

@@ -1,0 +1,71 @@
+"""Flexible CG with the two-grid preconditioner, whose products run on the fine
+lattice's 27-plane stencil: the smallest networks, lattices of odd extent that
+no block divides, several parts, a matrix that is symmetric to the bit (14
+planes read) and one that is not (27).  Against a sparse direct solve of the
+exported matrix: the iteration stops at a residual of 1e-10, so the solutions
+differ by at most the condition number (below 1e4 here) times that."""
+import ctypes
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as spl
+
+from gridap_amd import LearnedCoarseSolver, _lib, fpcg, problem_from_workload
+from gridap_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def matrix(prob, nparts):
+    rows, cols, vals = [], [], []
+    for q in range(nparts):
+        P = prob.export_part(q)
+        n = P["n_own"]
+        base = int(P["rowptr"][0])
+        ptr = P["rowptr"][: n + 1] - base
+        rows.append(np.repeat(P["row_gid"][:n], np.diff(ptr)))
+        cols.append(P["col_gid"][P["colidx"][: ptr[-1]] - base])
+        vals.append(P["val"][: ptr[-1]])
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    g0 = int(r.min())
+    return sp.coo_matrix((np.concatenate(vals), (r - g0, c - g0)), shape=(prob.ngdofs, prob.ngdofs)).tocsc()
+
+
+def change_entry(prob, factor):
+    """scale one off-diagonal entry of a middle row (single part)"""
+    P = prob.export_part(0)
+    base = int(P["rowptr"][0])
+    row = P["n_own"] // 2
+    k = int(P["rowptr"][row]) - base
+    if int(P["colidx"][k]) - base == row:
+        k += 1
+    ptr, nnz = ctypes.c_void_p(), ctypes.c_int64()
+    _lib.call("gdx_device_values", prob.handle, ctypes.byref(ptr), ctypes.byref(nnz))
+    v = np.array([P["val"][k] * factor])
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipMemcpy(ctypes.c_void_p(ptr.value + 8 * k), ctypes.c_void_p(v.ctypes.data), ctypes.c_size_t(8), 1) == 0
+
+
+@pytest.mark.parametrize("cells,parts,factor", [(8, (1, 1, 1), 1.0), (8, (1, 1, 1), 1.5), (16, (2, 3, 1), 1.0),
+                                                (16, (1, 1, 1), 1.5), (24, (3, 2, 2), 1.0), (24, (1, 1, 1), 0.5)])
+def test_fpcg_on_the_lattice_matches_direct_solve(gpu_ctx, cells, parts, factor):
+    assem, data = problem_from_workload(gpu_ctx, W.poisson3d_q1(cells, parts, rhs_const=0.0))
+    prob = assem._problem_for(data)
+    prob.cell_coefficient_grf(3, 0.1, 2.0)
+    prob.numeric()
+    prob.sync()
+    net = LearnedCoarseSolver(gpu_ctx, cells // 2, 1)
+    net.attach(prob)
+    net.set_options(2, use_network=False)
+    if factor != 1.0:
+        change_entry(prob, factor)  # after the attach: the solve takes the current values
+    A = matrix(prob, int(np.prod(parts)))
+    assert (abs(A - A.T).max() == 0.0) == (factor == 1.0)
+    rhs = np.random.default_rng(cells).normal(size=prob.ngdofs)
+    x, it, relres, _, fb = fpcg(prob, net, rhs, 1e-10)
+    assert not fb and relres <= 1.01e-10
+    ref = spl.spsolve(A, rhs)
+    assert np.linalg.norm(x - ref) <= 1e-6 * np.linalg.norm(ref)
+    net.close()
+    prob.close()
