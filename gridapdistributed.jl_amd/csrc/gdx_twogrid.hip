@@ -52,7 +52,7 @@ struct Level {
   int m = 0;
   double *cst = nullptr;  // Galerkin operator as a 27-point stencil [27][m^3]
   bool own_cst = true;    // false for the network grid (its stencil is TwoGrid::cst)
-  double *rhs = nullptr, *e = nullptr, *e2 = nullptr, *res = nullptr;  // [m^3]
+  double *rhs = nullptr, *e = nullptr, *e2 = nullptr;  // [m^3]
 };
 
 struct TwoGrid {
@@ -98,14 +98,15 @@ __global__ void k_gather(int ng, const long long *__restrict__ gn, const double 
 
 // rho[j] = dlat(2I) * sum_{|o|<=1} w(o) r(2I + o), I = j + 1, for interior coarse nodes; 0 on the padding plane
 __global__ void k_restrict(int n, int nf, const double *__restrict__ flat, const double *__restrict__ dlat,
-                           double *__restrict__ rho, double *__restrict__ rcoarse) {
-  const int64_t tot = (int64_t)n * n * n;
-  const int64_t j = blockIdx.x * (int64_t)kB + threadIdx.x;
+                           double *__restrict__ rho, double *__restrict__ rcoarse, double w,
+                           const double *__restrict__ cst, double *__restrict__ e) {
+  const unsigned tot = (unsigned)n * n * n, j = blockIdx.x * kB + threadIdx.x;
   if (j >= tot) return;
-  const int jx = (int)(j % n), jy = (int)((j / n) % n), jz = (int)(j / ((int64_t)n * n));
+  const int jx = (int)(j % n), jy = (int)(j / n % n), jz = (int)(j / ((unsigned)n * n));
   if (jx == n - 1 || jy == n - 1 || jz == n - 1) {
     rho[j] = 0.0;
     rcoarse[j] = 0.0;
+    if (e) e[j] = 0.0;
     return;
   }
   const int fx = 2 * (jx + 1), fy = 2 * (jy + 1), fz = 2 * (jz + 1);
@@ -117,6 +118,7 @@ __global__ void k_restrict(int n, int nf, const double *__restrict__ flat, const
         acc = fma(w, flat[(fx + ox) + (int64_t)nf * ((fy + oy) + (int64_t)nf * (fz + oz))], acc);
       }
   rcoarse[j] = acc;
+  if (e) e[j] = w * acc / cst[(size_t)13 * tot + j];  // the V-cycle's first damped-Jacobi sweep from zero
   rho[j] = acc * dlat[fx + (int64_t)nf * (fy + (int64_t)nf * fz)];
 }
 
@@ -452,25 +454,35 @@ __global__ void k_coarse_sweep(int n, double w, const double *__restrict__ cst, 
 }
 
 // fine lattice value of P ec (double coarse field on the network grid)
+// trilinear value at node (x, y, z) of a level of 2 mc cells from the interior
+// nodes of its coarse level: the 8 loads are predicated and issued together
+__device__ __forceinline__ double prolonged(int mc, int x, int y, int z, const double *__restrict__ ec) {
+  double v[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int kx = k & 1, ky = k >> 1 & 1, kz = k >> 2;
+    const int Jx = (x >> 1) + kx, Jy = (y >> 1) + ky, Jz = (z >> 1) + kz;
+    const bool in = kx <= (x & 1) && ky <= (y & 1) && kz <= (z & 1) && Jx >= 1 && Jy >= 1 && Jz >= 1 &&
+                    Jx <= mc - 1 && Jy <= mc - 1 && Jz <= mc - 1;
+    v[k] = in ? ec[(Jx - 1) + (int64_t)mc * ((Jy - 1) + (int64_t)mc * (Jz - 1))] : 0.0;
+  }
+  const double w = ((x & 1) ? 0.5 : 1.0) * ((y & 1) ? 0.5 : 1.0) * ((z & 1) ? 0.5 : 1.0);
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) acc = fma(w, v[k], acc);
+  return acc;
+}
+
+// (32-bit node numbers: a lattice of 2^31 nodes would need a 464 GB stencil)
 __global__ void k_prolong_d(int n, int nf, const double *__restrict__ ec, double *__restrict__ flat) {
-  const int64_t tot = (int64_t)nf * nf * nf;
-  const int64_t i = blockIdx.x * (int64_t)kB + threadIdx.x;
+  const unsigned tot = (unsigned)nf * nf * nf, i = blockIdx.x * kB + threadIdx.x;
   if (i >= tot) return;
-  const int x = (int)(i % nf), y = (int)((i / nf) % nf), z = (int)(i / ((int64_t)nf * nf));
+  const int x = (int)(i % nf), y = (int)(i / nf % nf), z = (int)(i / ((unsigned)nf * nf));
   if (x == 0 || y == 0 || z == 0 || x == nf - 1 || y == nf - 1 || z == nf - 1) {
     flat[i] = 0.0;
     return;
   }
-  double acc = 0.0;
-  for (int kz = 0; kz < 1 + (z & 1); ++kz)
-    for (int ky = 0; ky < 1 + (y & 1); ++ky)
-      for (int kx = 0; kx < 1 + (x & 1); ++kx) {
-        const int Ix = (x >> 1) + kx, Iy = (y >> 1) + ky, Iz = (z >> 1) + kz;
-        if (Ix < 1 || Iy < 1 || Iz < 1 || Ix > n - 1 || Iy > n - 1 || Iz > n - 1) continue;
-        const double w = ((x & 1) ? 0.5 : 1.0) * ((y & 1) ? 0.5 : 1.0) * ((z & 1) ? 0.5 : 1.0);
-        acc = fma(w, ec[(Ix - 1) + (int64_t)n * ((Iy - 1) + (int64_t)n * (Iz - 1))], acc);
-      }
-  flat[i] = acc;
+  flat[i] = prolonged(n, x, y, z, ec);
 }
 
 // ---------------------------------------------------------------------------
@@ -507,47 +519,118 @@ __global__ void k_sweep0(int m, double w, const double *__restrict__ cst, const 
   e[j] = padding(j, m, jx, jy, jz) ? 0.0 : w * rhs[j] / cst[13 * tot + j];
 }
 
-// full weighting from level mf to mf/2: rc[J] = sum_o w(o) r[2J + o]
-__global__ void k_restrict_c(int mf, const double *__restrict__ rf, double *__restrict__ rc) {
+// full weighting from level mf to mf/2: rc[J] = sum_o w(o) r[2J + o], and that
+// level's first damped-Jacobi sweep from zero, ec = w Dc^-1 rc (ec null: the
+// coarsest level, which starts its own)
+__global__ void k_restrict_c(int mf, double w, const double *__restrict__ rf, const double *__restrict__ ccst,
+                             double *__restrict__ rc, double *__restrict__ ec) {
   const int mc = mf / 2;
-  const int64_t tot = (int64_t)mc * mc * mc;
-  const int64_t j = blockIdx.x * (int64_t)kB + threadIdx.x;
+  const unsigned tot = (unsigned)mc * mc * mc, j = blockIdx.x * kB + threadIdx.x;
   if (j >= tot) return;
-  int jx, jy, jz;
-  if (padding(j, mc, jx, jy, jz)) {
-    rc[j] = 0.0;
-    return;
+  const int jx = (int)(j % mc), jy = (int)(j / mc % mc), jz = (int)(j / ((unsigned)mc * mc));
+  double acc = 0.0, e0 = 0.0;
+  if (jx < mc - 1 && jy < mc - 1 && jz < mc - 1) {
+    for (int oz = 0; oz < 3; ++oz)  // storage of the fine nodes 2J + o: 2j .. 2j + 2
+      for (int oy = 0; oy < 3; ++oy)
+        for (int ox = 0; ox < 3; ++ox) {
+          const double wt = (ox != 1 ? 0.5 : 1.0) * (oy != 1 ? 0.5 : 1.0) * (oz != 1 ? 0.5 : 1.0);
+          acc = fma(wt, rf[(2 * jx + ox) + (size_t)mf * ((2 * jy + oy) + (size_t)mf * (2 * jz + oz))], acc);
+        }
+    if (ec) e0 = w * acc / ccst[(size_t)13 * tot + j];
   }
-  const int fx = 2 * (jx + 1) - 1, fy = 2 * (jy + 1) - 1, fz = 2 * (jz + 1) - 1;  // storage of fine node 2J
-  double acc = 0.0;
-  for (int oz = -1; oz <= 1; ++oz)
-    for (int oy = -1; oy <= 1; ++oy)
-      for (int ox = -1; ox <= 1; ++ox) {
-        const double w = (ox ? 0.5 : 1.0) * (oy ? 0.5 : 1.0) * (oz ? 0.5 : 1.0);
-        acc = fma(w, rf[(fx + ox) + (int64_t)mf * ((fy + oy) + (int64_t)mf * (fz + oz))], acc);
-      }
   rc[j] = acc;
+  if (ec) ec[j] = e0;
 }
 
-// ef += P ec (trilinear, from level mf/2 to mf)
-__global__ void k_prolong_add_c(int mf, const double *__restrict__ ec, double *__restrict__ ef) {
-  const int mc = mf / 2;
-  const int64_t tot = (int64_t)mf * mf * mf;
-  const int64_t i = blockIdx.x * (int64_t)kB + threadIdx.x;
-  if (i >= tot) return;
-  int ix, iy, iz;
-  if (padding(i, mf, ix, iy, iz)) return;
-  const int x = ix + 1, y = iy + 1, z = iz + 1;  // fine node
-  double acc = 0.0;
-  for (int kz = 0; kz < 1 + (z & 1); ++kz)
-    for (int ky = 0; ky < 1 + (y & 1); ++ky)
-      for (int kx = 0; kx < 1 + (x & 1); ++kx) {
-        const int Jx = (x >> 1) + kx, Jy = (y >> 1) + ky, Jz = (z >> 1) + kz;
-        if (Jx < 1 || Jy < 1 || Jz < 1 || Jx > mc - 1 || Jy > mc - 1 || Jz > mc - 1) continue;
-        const double w = ((x & 1) ? 0.5 : 1.0) * ((y & 1) ? 0.5 : 1.0) * ((z & 1) ? 0.5 : 1.0);
-        acc = fma(w, ec[(Jx - 1) + (int64_t)mc * ((Jy - 1) + (int64_t)mc * (Jz - 1))], acc);
-      }
-  ef[i] += acc;
+// The residual rhs - A e and k_restrict_c's work in one launch, for levels up to
+// kDownMax.  A workgroup owns 16 x 2 x 2 coarse nodes and keeps the residual at
+// the 33 x 5 x 5 fine nodes below them in LDS, 1.6 of them per own node.  Small
+// levels are bound by the launch and one round of loads: 7.5 us against 14 for
+// residual, weighting and sweep apart at 8^3 to 32^3.  Where the planes' bytes
+// bound the residual the extra nodes cost more than the launches: at 64^3 29 us
+// against 15 for k_resid and k_restrict_c.
+constexpr int kDownMax = 32;
+constexpr int kDnX = 16, kDnY = 2, kDnZ = 2, kDnThreads = 832;
+__global__ __launch_bounds__(kDnThreads) void k_down(int m, double w, const double *__restrict__ cst,
+                                                     const double *__restrict__ rhs, const double *__restrict__ e,
+                                                     const double *__restrict__ ccst, double *__restrict__ rc,
+                                                     double *__restrict__ ec) {
+  constexpr int FX = 2 * kDnX + 1, FY = 2 * kDnY + 1, FZ = 2 * kDnZ + 1;
+  __shared__ double res[FX * FY * FZ];
+  const int mc = m / 2, t = threadIdx.x;
+  const int X0 = kDnX * blockIdx.x, Y0 = kDnY * blockIdx.y, Z0 = kDnZ * blockIdx.z;
+  const int64_t tot = (int64_t)m * m * m, totc = (int64_t)mc * mc * mc;
+  // coarse storage index J has fine storage nodes 2J .. 2J + 2
+  for (int q = t; q < FX * FY * FZ; q += kDnThreads) {
+    const int x = 2 * X0 + q % FX, y = 2 * Y0 + (q / FX) % FY, z = 2 * Z0 + q / (FX * FY);
+    double r = 0.0;
+    if (x <= m - 2 && y <= m - 2 && z <= m - 2) {
+      const int64_t j = x + (int64_t)m * (y + (int64_t)m * z);
+      r = stencil_residual(rhs[j], m, tot, j, x, y, z, cst, e);
+    }
+    res[q] = r;
+  }
+  __syncthreads();
+  if (t >= kDnX * kDnY * kDnZ) return;
+  const int lx = t % kDnX, ly = (t / kDnX) % kDnY, lz = t / (kDnX * kDnY);
+  const int X = X0 + lx, Y = Y0 + ly, Z = Z0 + lz;
+  if (X >= mc || Y >= mc || Z >= mc) return;
+  const int64_t j = X + (int64_t)mc * (Y + (int64_t)mc * Z);
+  double acc = 0.0, e0 = 0.0;
+  if (X < mc - 1 && Y < mc - 1 && Z < mc - 1) {
+    for (int oz = 0; oz < 3; ++oz)
+      for (int oy = 0; oy < 3; ++oy)
+        for (int ox = 0; ox < 3; ++ox) {
+          const double wt = (ox != 1 ? 0.5 : 1.0) * (oy != 1 ? 0.5 : 1.0) * (oz != 1 ? 0.5 : 1.0);
+          acc = fma(wt, res[2 * lx + ox + FX * (2 * ly + oy + FY * (2 * lz + oz))], acc);
+        }
+    if (ec) e0 = w * acc / ccst[13 * totc + j];
+  }
+  rc[j] = acc;
+  if (ec) ec[j] = e0;
+}
+
+// One launch up a level: a' = a + P ec (trilinear, from level m/2) and one
+// damped-Jacobi sweep, b = a' + w D^-1 (rhs - A a').  A workgroup owns 16 x 4 x 4
+// nodes and keeps a' there and on the layer around them in LDS.
+constexpr int kUpX = 16, kUpY = 4, kUpZ = 4, kUpThreads = kUpX * kUpY * kUpZ;
+__global__ __launch_bounds__(kUpThreads) void k_up(int m, double w, const double *__restrict__ cst,
+                                                   const double *__restrict__ rhs, const double *__restrict__ a,
+                                                   const double *__restrict__ ec, double *__restrict__ b) {
+  constexpr int HX = kUpX + 2, HY = kUpY + 2, HZ = kUpZ + 2;
+  __shared__ double ap[HX * HY * HZ];
+  const int mc = m / 2, t = threadIdx.x;
+  const int64_t tot = (int64_t)m * m * m;
+  const int X0 = kUpX * blockIdx.x, Y0 = kUpY * blockIdx.y, Z0 = kUpZ * blockIdx.z;
+  const int lx = t % kUpX, ly = (t / kUpX) % kUpY, lz = t / (kUpX * kUpY);
+  const int X = X0 + lx, Y = Y0 + ly, Z = Z0 + lz;
+  const bool live = X <= m - 2 && Y <= m - 2 && Z <= m - 2;
+  const int64_t j = live ? X + (int64_t)m * (Y + (int64_t)m * Z) : 0;
+  // the node's coefficients (zero towards the boundary) load while a' is formed
+  double cv[27];
+#pragma unroll
+  for (int k = 0; k < 27; ++k) cv[k] = live ? cst[k * tot + j] : 0.0;
+  const double r0 = live ? rhs[j] : 0.0;
+  for (int q = t; q < HX * HY * HZ; q += kUpThreads) {
+    const int ix = X0 + q % HX - 1, iy = Y0 + (q / HX) % HY - 1, iz = Z0 + q / (HX * HY) - 1;
+    double v = 0.0;
+    if (ix >= 0 && iy >= 0 && iz >= 0 && ix <= m - 2 && iy <= m - 2 && iz <= m - 2) {
+      v = a[ix + (int64_t)m * (iy + (int64_t)m * iz)] + prolonged(mc, ix + 1, iy + 1, iz + 1, ec);
+    }
+    ap[q] = v;
+  }
+  __syncthreads();
+  if (X >= m || Y >= m || Z >= m) return;
+  const int64_t js = X + (int64_t)m * (Y + (int64_t)m * Z);
+  if (!live) {
+    b[js] = 0.0;
+    return;
+  }
+  const int c = (lx + 1) + HX * ((ly + 1) + HY * (lz + 1));
+  double r = r0;
+#pragma unroll
+  for (int k = 0; k < 27; ++k) r -= cv[k] * ap[c + (k % 3 - 1) + HX * (((k / 3) % 3 - 1) + HY * (k / 9 - 1))];
+  b[js] = ap[c] + w * r / cv[13];
 }
 
 // coarsest level (m <= 8): damped-Jacobi sweeps from zero in one workgroup;
@@ -618,6 +701,61 @@ __global__ __launch_bounds__(kCoarsestThreads) void k_coarsest(int m, double w, 
     b = tmp;
   }
   if (sub == 0 && j < tot) e[j] = a[j];
+}
+
+// the same sweeps where one wave holds the level (m <= 5: at most 64 interior
+// points, where halving stops for 2^k and 3 2^k): L lanes per point, the grid in
+// LDS with a zero layer around it, the point's lanes summed by lane moves.  A
+// sweep is one chain of LDS reads, multiply-adds and a write, without a barrier
+// between waves.
+constexpr int kWaveLevel = 5;
+template <int CTRL>
+__device__ __forceinline__ double lane_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+template <int L>
+__global__ __launch_bounds__(64) void k_coarsest_wave(int m, double w, int sweeps, const double *__restrict__ cst,
+                                                      const double *__restrict__ rhs, double *__restrict__ e) {
+  constexpr int KL = (27 + L - 1) / L, M = kWaveLevel + 1;
+  __shared__ double g[2][M * M * M];
+  const int t = threadIdx.x, p = t / L, sub = t % L, mi = m - 1, tot = m * m * m;
+  const bool live = p < mi * mi * mi;
+  const int jx = live ? p % mi : 0, jy = live ? (p / mi) % mi : 0, jz = live ? p / (mi * mi) : 0;
+  const int j = jx + m * (jy + m * jz), c = (jx + 1) + M * ((jy + 1) + M * (jz + 1));
+  for (int i = t; i < 2 * M * M * M; i += 64) (&g[0][0])[i] = 0.0;
+  for (int i = t; i < tot; i += 64) e[i] = 0.0;  // the padding; the points follow at the end
+  double cf[KL];
+  int of[KL];
+#pragma unroll
+  for (int i = 0; i < KL; ++i) {
+    const int k = sub + L * i;
+    cf[i] = live && k < 27 ? cst[k * tot + j] : 0.0;  // zero towards the boundary
+    of[i] = k < 27 ? c + (k % 3 - 1) + M * ((k / 3) % 3 - 1) + M * M * (k / 9 - 1) : c;
+  }
+  const double rj = live ? rhs[j] : 0.0, wd = live ? w / cst[13 * tot + j] : 0.0;
+  double a = 0.0;
+  __syncthreads();
+  for (int s = 0; s < sweeps; ++s) {
+    double v[KL], p0 = 0.0, p1 = 0.0;
+#pragma unroll
+    for (int i = 0; i < KL; ++i) v[i] = g[s & 1][of[i]];
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+      if (i & 1) p1 = fma(cf[i], v[i], p1);
+      else p0 = fma(cf[i], v[i], p0);
+    }
+    double part = p0 + p1;
+    if (L >= 2) part += lane_move<0xB1>(part);   // lane ^ 1
+    if (L >= 4) part += lane_move<0x4E>(part);   // lane ^ 2
+    if (L >= 8) part += lane_move<0x141>(part);  // the other four of eight
+    a = fma(wd, rj - part, a);
+    if (sub == 0 && live) g[(s & 1) ^ 1][c] = a;
+    __syncthreads();
+  }
+  if (sub == 0 && live) e[j] = a;
 }
 
 // partial sums of squares (and of a*b) over a grid-stride slice
@@ -725,13 +863,6 @@ __global__ void k_add(int n, double *__restrict__ z, const double *__restrict__ 
   const int i = blockIdx.x * kB + threadIdx.x;
   if (i < n) z[i] += c[i];
 }
-// z += w D^-1 (r - t), t = A z
-__global__ void k_jacobi_post(int n, double w, const double *__restrict__ dinv, const double *__restrict__ r,
-                              const double *__restrict__ t, double *__restrict__ z) {
-  const int i = blockIdx.x * kB + threadIdx.x;
-  if (i < n) z[i] = fma(w * dinv[i], r[i] - t[i], z[i]);
-}
-
 __host__ __device__ inline uint64_t mix64(uint64_t z) {
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
   z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
@@ -914,15 +1045,17 @@ void lattice_product(TwoGrid *T, const double *x, const double *r, double *y, hi
 }
 
 // network input from a fine residual in global-id order, or on the lattice (s
-// into red[kS]); with the network off only the coarse residual rc is formed
-void make_input(gdx_nn *nn, TwoGrid *T, const double *r, hipStream_t st, bool for_net = true, bool lattice = false) {
+// into red[kS]); with the network off only the coarse residual rc is formed, and
+// with e0 the V-cycle's first sweep for it
+void make_input(gdx_nn *nn, TwoGrid *T, const double *r, hipStream_t st, bool for_net = true, bool lattice = false,
+                double *e0 = nullptr) {
   nn::Net &N = nn->net;
   const int64_t v = (int64_t)T->n * T->n * T->n;
   // restriction reads only interior lattice nodes, all of which the scatter
   // writes: no clearing (and no memset, so this can be captured in a graph)
   if (!lattice) hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, T->flat);
   hipLaunchKernelGGL(k_restrict, dim3(nb(v)), dim3(kB), 0, st, T->n, T->nf, lattice ? r : T->flat, T->dlat, T->rho,
-                     T->rc);
+                     T->rc, kOmegaC, T->cst, e0);
   if (!for_net) return;
   rms(T, T->rho, nullptr, v, T->red + kS, 0, st);
   hipLaunchKernelGGL(k_input0, dim3(nb(v)), dim3(kB), 0, st, v, T->rho, T->red + kS, N.inp_f);
@@ -931,7 +1064,7 @@ void make_input(gdx_nn *nn, TwoGrid *T, const double *r, hipStream_t st, bool fo
 
 void mg_free(TwoGrid *T) {
   for (Level &L : T->lv) {
-    void *ptrs[] = {L.own_cst ? L.cst : nullptr, L.rhs, L.e, L.e2, L.res};
+    void *ptrs[] = {L.own_cst ? L.cst : nullptr, L.rhs, L.e, L.e2};
     for (void *q : ptrs)
       if (q) (void)hipFree(q);
   }
@@ -954,8 +1087,7 @@ int mg_setup(TwoGrid *T, hipStream_t st) {
       Level &M = T->lv.back();
       bool ok = hipMalloc(reinterpret_cast<void **>(&M.rhs), v * sizeof(double)) == hipSuccess &&
                 hipMalloc(reinterpret_cast<void **>(&M.e), v * sizeof(double)) == hipSuccess &&
-                hipMalloc(reinterpret_cast<void **>(&M.e2), v * sizeof(double)) == hipSuccess &&
-                hipMalloc(reinterpret_cast<void **>(&M.res), v * sizeof(double)) == hipSuccess;
+                hipMalloc(reinterpret_cast<void **>(&M.e2), v * sizeof(double)) == hipSuccess;
       if (l == 0) {
         M.cst = T->cst;
         M.own_cst = false;
@@ -975,39 +1107,55 @@ int mg_setup(TwoGrid *T, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-// V-cycle on level l for the right-hand side lv[l].rhs, from a zero guess:
+// V-cycle on level l for the right-hand side rhs, from a zero guess whose first
+// sweep is already in lv[l].e (not on the coarsest level):
 // nu damped-Jacobi sweeps, coarse-grid correction, nu sweeps (the coarsest
 // level: sweeps in one workgroup).  Returns the buffer holding the correction.
-double *vcycle(TwoGrid *T, size_t l, hipStream_t st) {
+double *vcycle(TwoGrid *T, size_t l, const double *rhs, hipStream_t st) {
   Level &L = T->lv[l];
   const int64_t v = (int64_t)L.m * L.m * L.m;
   if (l + 1 == T->lv.size()) {
-    switch (coarsest_lanes(L.m * L.m * L.m)) {  // m <= 8: 2 to 32 lanes per point
+    const int np = (L.m - 1) * (L.m - 1) * (L.m - 1);
+    if (L.m <= kWaveLevel) {
+      hipLaunchKernelGGL(np <= 8 ? k_coarsest_wave<8> : np <= 32 ? k_coarsest_wave<2> : k_coarsest_wave<1>, dim3(1),
+                         dim3(64), 0, st, L.m, kOmegaC, T->coarsest_sweeps, L.cst, rhs, L.e);
+      return L.e;
+    }
+    switch (coarsest_lanes(L.m * L.m * L.m)) {  // 6 <= m <= 8: 2 or 4 lanes per point
 #define GDX_COARSEST(NL)                                                                                           \
   case NL:                                                                                                         \
     hipLaunchKernelGGL(k_coarsest<NL>, dim3(1), dim3(kCoarsestThreads), 0, st, L.m, kOmegaC, T->coarsest_sweeps, \
-                       L.cst, L.rhs, L.e);                                                                         \
+                       L.cst, rhs, L.e);                                                                           \
     break;
-      GDX_COARSEST(2) GDX_COARSEST(4) GDX_COARSEST(8) GDX_COARSEST(16) GDX_COARSEST(32)
+      GDX_COARSEST(2) GDX_COARSEST(4)
 #undef GDX_COARSEST
       default: break;
     }
     return L.e;
   }
   double *a = L.e, *b = L.e2;
-  hipLaunchKernelGGL(k_sweep0, dim3(nb(v)), dim3(kB), 0, st, L.m, kOmegaC, L.cst, L.rhs, a);
   for (int k = 1; k < T->nu; ++k) {
-    hipLaunchKernelGGL(k_coarse_sweep, dim3(nb(v)), dim3(kB), 0, st, L.m, kOmegaC, L.cst, L.rhs, a, b);
+    hipLaunchKernelGGL(k_coarse_sweep, dim3(nb(v)), dim3(kB), 0, st, L.m, kOmegaC, L.cst, rhs, a, b);
     std::swap(a, b);
   }
-  hipLaunchKernelGGL(k_resid, dim3(nb(v)), dim3(kB), 0, st, L.m, L.cst, L.rhs, a, L.res);
   Level &C = T->lv[l + 1];
-  const int64_t vc = (int64_t)C.m * C.m * C.m;
-  hipLaunchKernelGGL(k_restrict_c, dim3(nb(vc)), dim3(kB), 0, st, L.m, L.res, C.rhs);
-  const double *c = vcycle(T, l + 1, st);
-  hipLaunchKernelGGL(k_prolong_add_c, dim3(nb(v)), dim3(kB), 0, st, L.m, c, a);
-  for (int k = 0; k < T->nu; ++k) {
-    hipLaunchKernelGGL(k_coarse_sweep, dim3(nb(v)), dim3(kB), 0, st, L.m, kOmegaC, L.cst, L.rhs, a, b);
+  const bool last = l + 2 == T->lv.size();
+  const auto per = [](int n, int w) { return (unsigned)((n + w - 1) / w); };
+  double *e0 = last ? nullptr : C.e;
+  if (L.m > kDownMax) {
+    hipLaunchKernelGGL(k_resid, dim3(nb(v)), dim3(kB), 0, st, L.m, L.cst, rhs, a, b);
+    hipLaunchKernelGGL(k_restrict_c, dim3(nb((int64_t)C.m * C.m * C.m)), dim3(kB), 0, st, L.m, kOmegaC, b, C.cst,
+                       C.rhs, e0);
+  } else {
+    hipLaunchKernelGGL(k_down, dim3(per(C.m, kDnX), per(C.m, kDnY), per(C.m, kDnZ)), dim3(kDnThreads), 0, st, L.m,
+                       kOmegaC, L.cst, rhs, a, C.cst, C.rhs, e0);
+  }
+  const double *c = vcycle(T, l + 1, C.rhs, st);
+  hipLaunchKernelGGL(k_up, dim3(per(L.m, kUpX), per(L.m, kUpY), per(L.m, kUpZ)), dim3(kUpThreads), 0, st, L.m,
+                     kOmegaC, L.cst, rhs, a, c, b);
+  std::swap(a, b);
+  for (int k = 1; k < T->nu; ++k) {
+    hipLaunchKernelGGL(k_coarse_sweep, dim3(nb(v)), dim3(kB), 0, st, L.m, kOmegaC, L.cst, rhs, a, b);
     std::swap(a, b);
   }
   return a;
@@ -1165,12 +1313,18 @@ int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
 static int coarse_correction(gdx_nn *nn, TwoGrid *T, const double *s, bool lattice, double *flat, hipStream_t st) {
   nn::Net &N = nn->net;
   const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
-  make_input(nn, T, s, st, T->use_net, lattice);
+  const bool mg = T->mg && T->lv.size() > 1;
+  make_input(nn, T, s, st, T->use_net, lattice, mg && !T->use_net ? T->lv[0].e : nullptr);
   if (T->use_net) {
     int rc = N.forward_dev();
     if (rc) return rc;
   }
   const int64_t v = (int64_t)T->n * T->n * T->n;
+  if (mg && !T->use_net) {  // from the zero guess: the V-cycle on rc itself
+    const double *d = vcycle(T, 0, T->rc, st);
+    hipLaunchKernelGGL(k_prolong_d, dim3(nb(nfl)), dim3(kB), 0, st, T->n, T->nf, d, flat);
+    return GDX_OK;
+  }
   hipLaunchKernelGGL(k_out_to_coarse, dim3(nb(v)), dim3(kB), 0, st, T->n, N.out, T->red + kS, T->use_net ? 1 : 0,
                      T->ca);
   if (T->use_net) {
@@ -1182,10 +1336,12 @@ static int coarse_correction(gdx_nn *nn, TwoGrid *T, const double *s, bool latti
     hipLaunchKernelGGL(k_scale_by, dim3(nb(v)), dim3(kB), 0, st, v, T->red + kS + 6, T->ca);
   }
   double *ea = T->ca, *eb = T->cb;
-  if (T->mg && T->lv.size() > 1) {
-    // V-cycle on the coarse residual of the (network's or zero) guess
-    hipLaunchKernelGGL(k_resid, dim3(nb(v)), dim3(kB), 0, st, T->n, T->cst, T->rc, ea, T->lv[0].rhs);
-    const double *d = vcycle(T, 0, st);
+  if (mg) {
+    // V-cycle on the coarse residual of the network's guess
+    const Level &L = T->lv[0];
+    hipLaunchKernelGGL(k_resid, dim3(nb(v)), dim3(kB), 0, st, T->n, T->cst, T->rc, ea, L.rhs);
+    hipLaunchKernelGGL(k_sweep0, dim3(nb(v)), dim3(kB), 0, st, T->n, kOmegaC, T->cst, L.rhs, L.e);
+    const double *d = vcycle(T, 0, L.rhs, st);
     hipLaunchKernelGGL(k_add, dim3(nb(v)), dim3(kB), 0, st, (int)v, ea, d);
   } else {
     for (int k = 0; k < T->sweeps; ++k) {

@@ -11,6 +11,7 @@ import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spl
 
+from coarse_bound import Multilevel
 from gridap_amd import LearnedCoarseSolver, _lib, fpcg, problem_from_workload
 from gridap_amd import workloads as W
 
@@ -67,5 +68,38 @@ def test_fpcg_on_the_lattice_matches_direct_solve(gpu_ctx, cells, parts, factor)
     assert not fb and relres <= 1.01e-10
     ref = spl.spsolve(A, rhs)
     assert np.linalg.norm(x - ref) <= 1e-6 * np.linalg.norm(ref)
+    net.close()
+    prob.close()
+
+
+# networks of 8 to 40 cells: a level of three to seven cells at the bottom (one
+# wave up to five, else a workgroup), levels that the 16 x 2 x 2 and 16 x 4 x 4
+# node tiles do not divide, and one above 32 whose residual is a launch of its own
+@pytest.mark.parametrize("n,nu", [(8, 1), (12, 3), (20, 1), (24, 2), (28, 2), (32, 1), (40, 2)])
+def test_vcycle_matches_reference(gpu_ctx, n, nu):
+    cells = 2 * n
+    assem, data = problem_from_workload(gpu_ctx, W.poisson3d_q1(cells, (1, 1, 1), rhs_const=0.0))
+    prob = assem._problem_for(data)
+    prob.cell_coefficient_grf(5, 0.1, 2.0)
+    prob.numeric()
+    prob.sync()
+    net = LearnedCoarseSolver(gpu_ctx, n, 1)
+    net.attach(prob)
+    net.set_options(8, use_network=False)
+    assert net.set_multigrid(True, nu) > 1
+    P = prob.export_part(0)
+    A = matrix(prob, 1).tocsr()
+    # free ids by lattice node, x fastest
+    order = P["ldof_gid"][np.argsort(P["ldof_gnode"])] - P["ldof_gid"].min()
+    A = A[order][:, order]
+    bottom = n
+    while bottom % 2 == 0 and bottom > 4:
+        bottom //= 2
+    ref = Multilevel(A, cells, nu=nu, coarsest_cells=bottom)
+    r = np.random.default_rng(n).normal(size=prob.ngdofs)
+    z = net.apply(r)[order]
+    zr = ref(r[order])
+    # rounding of 27 products a sweep, about 100 sweeps deep (1e-12), times the spread of the diagonals (about 1e2)
+    assert np.linalg.norm(z - zr) <= 1e-10 * np.linalg.norm(zr)
     net.close()
     prob.close()
