@@ -323,12 +323,12 @@ struct FpcgPrec {
   void *ctx;
   // the iteration on the preconditioner's own lattice (nullptr: none): begin
   // takes the matrix's current values (unless current: the preconditioner was
-  // just built from them) and puts r there; n entries, with the operator and
-  // the preconditioner between lattice vectors; end puts x back
-  int (*begin)(void *ctx, const double *r, bool current, int *n, double *vecs[5], hipStream_t st) = nullptr;
-  void (*product)(void *ctx, const double *x, double *y, hipStream_t st) = nullptr;
-  int (*apply_lattice)(void *ctx, const double *r, double *z, hipStream_t st) = nullptr;
-  void (*end)(void *ctx, const double *x_lattice, double *x, hipStream_t st) = nullptr;
+  // just built from them), x = 0 and the residual r; first sets p = M r; iterate
+  // makes one step with sc = {p.q, p.r, z.q, r.r}; end puts x back
+  int (*begin)(void *ctx, const double *r, bool current, hipStream_t st) = nullptr;
+  int (*first)(void *ctx, hipStream_t st) = nullptr;
+  int (*iterate)(void *ctx, double *sc, hipStream_t st) = nullptr;
+  void (*end)(void *ctx, double *x, hipStream_t st) = nullptr;
   bool current = false;
 };
 int solve_fpcg(gdx_problem *p, const FpcgPrec *prec, const double *rhs_h, double rtol, int maxiter, double *xh,

@@ -403,10 +403,9 @@ static void spmv(gdx_problem *p, SolveData *s, const double *x, double *y, hipSt
 }
 
 static void dot2(SolveData *s, const double *a, const double *b, const double *c, const double *d, double *out,
-                 hipStream_t st, int n = -1) {
-  if (n < 0) n = s->n;
-  const int nb = std::min(kRedBlocks, std::max(1, (n + kBlk - 1) / kBlk));
-  hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(kBlk), 0, st, n, a, b, c, d, s->part);
+                 hipStream_t st) {
+  const int nb = std::min(kRedBlocks, std::max(1, (s->n + kBlk - 1) / kBlk));
+  hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(kBlk), 0, st, s->n, a, b, c, d, s->part);
   hipLaunchKernelGGL(k_finish2, dim3(1), dim3(kBlk), 0, st, s->part, nb, out);
 }
 
@@ -607,23 +606,12 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
     hipLaunchKernelGGL(k_gather_b, g, b, 0, st, n, s->bidx, p->dev.b, s->b);
   }
   hipLaunchKernelGGL(k_inv_diag, g, b, 0, st, n, s->dpos, p->dev.values, s->dinv);
-  // the iteration's vectors: global-id order, or the preconditioner's lattice
-  double *vx = s->x, *vr = s->r, *vz = s->z, *vp = s->p, *vq = s->q;
-  int nv = n;
+  (void)hipMemsetAsync(s->x, 0, n * sizeof(double), st);
   if (prec->begin) {
-    double *v[5];
-    if ((rc = prec->begin(prec->ctx, s->b, prec->current, &nv, v, st))) return rc;
-    vx = v[0], vr = v[1], vz = v[2], vp = v[3], vq = v[4];
-  } else if (hipMemcpyAsync(vr, s->b, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
+    if ((rc = prec->begin(prec->ctx, s->b, prec->current, st))) return rc;
+  } else if (hipMemcpyAsync(s->r, s->b, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
     return GDX_ERR_HIP;
   }
-  const dim3 gv((nv + kBlk - 1) / kBlk);
-  auto product = [&](const double *x, double *y) {
-    if (prec->begin) prec->product(prec->ctx, x, y, st);
-    else spmv(p, s, x, y, st);
-  };
-  const auto apply = prec->begin ? prec->apply_lattice : prec->apply;
-  (void)hipMemsetAsync(vx, 0, nv * sizeof(double), st);
   dot2(s, s->b, s->b, nullptr, nullptr, s->sc + 6, st);
   double bb;
   if (hipMemcpyAsync(&bb, s->sc + 6, sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -633,18 +621,24 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
   bool fall = false, nonfinite = false;
   double last_check = bnorm;
   if (bnorm > 0.0) {
-    if ((rc = apply(prec->ctx, vr, vz, st))) return rc;
-    if (hipMemcpyAsync(vp, vz, nv * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) return GDX_ERR_HIP;
+    if (prec->begin) {
+      if ((rc = prec->first(prec->ctx, st))) return rc;
+    } else {
+      if ((rc = prec->apply(prec->ctx, s->r, s->z, st))) return rc;
+      if (hipMemcpyAsync(s->p, s->z, n * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess)
+        return GDX_ERR_HIP;
+    }
     IterGraph G;
     for (it = 1; it <= maxiter; ++it) {
       rc = run_iteration(st, G, [&]() {
-        product(vp, vq);
-        dot2(s, vp, vq, vp, vr, s->sc, st, nv);  // sc[0] = pq, sc[1] = pr
-        hipLaunchKernelGGL(k_fcg_update, gv, b, 0, st, nv, s->sc, vx, vr, vp, vq);
-        int r2 = apply(prec->ctx, vr, vz, st);
+        if (prec->begin) return prec->iterate(prec->ctx, s->sc, st);
+        spmv(p, s, s->p, s->q, st);
+        dot2(s, s->p, s->q, s->p, s->r, s->sc, st);  // sc[0] = pq, sc[1] = pr
+        hipLaunchKernelGGL(k_fcg_update, g, b, 0, st, n, s->sc, s->x, s->r, s->p, s->q);
+        int r2 = prec->apply(prec->ctx, s->r, s->z, st);
         if (r2) return r2;
-        dot2(s, vz, vq, vr, vr, s->sc + 2, st, nv);  // sc[2] = zq, sc[3] = rr
-        hipLaunchKernelGGL(k_fcg_dir, gv, b, 0, st, nv, s->sc, vz, vp);
+        dot2(s, s->z, s->q, s->r, s->r, s->sc + 2, st);  // sc[2] = zq, sc[3] = rr
+        hipLaunchKernelGGL(k_fcg_dir, g, b, 0, st, n, s->sc, s->z, s->p);
         return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
       });
       if (rc) return rc;
@@ -673,7 +667,7 @@ static int fpcg_run(gdx_problem *p, SolveData *s, const FpcgPrec *prec, const do
     }
     if (it > maxiter) it = maxiter;
   }
-  if (prec->begin) prec->end(prec->ctx, vx, s->x, st);
+  if (prec->begin) prec->end(prec->ctx, s->x, st);
   if (fall) {
     // Jacobi-PCG from the current iterate (or from zero if it is not finite);
     // s->b still holds the right-hand side

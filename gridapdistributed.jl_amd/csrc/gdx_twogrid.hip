@@ -1000,6 +1000,29 @@ __global__ __launch_bounds__(kB) void k_asymmetric(int nf, const double *__restr
   if (__syncthreads_or(bad) && threadIdx.x == 0) *asym = 1;
 }
 
+// the workgroup's sums of a and b into part[blk] and part[nblk + blk]
+__device__ __forceinline__ void block_dots(double a, double b, int blk, int nblk, double *__restrict__ part) {
+  __shared__ double sh[2][kB / 64];
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o);
+    b += __shfl_xor(b, o);
+  }
+  if (threadIdx.x % 64 == 0) {
+    sh[0][threadIdx.x / 64] = a;
+    sh[1][threadIdx.x / 64] = b;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  a = sh[0][0];
+  b = sh[1][0];
+  for (int k = 1; k < kB / 64; ++k) {
+    a += sh[0][k];
+    b += sh[1][k];
+  }
+  part[blk] = a;
+  part[nblk + blk] = b;
+}
+
 // y = A x on the fine lattice (boundary nodes 0), or y = r - A x.  A is the
 // 27-plane stencil fst; where it is symmetric only its upper 14 planes are
 // read, the lower offsets' coefficients being the upper ones of the neighbour,
@@ -1008,40 +1031,108 @@ __global__ __launch_bounds__(kB) void k_asymmetric(int nf, const double *__restr
 // for the CSR product with 16-bit column codes, and no gather through ids.
 // 128^3 cells: 80 us (the CSR product 144); 96^3: 25 us, its planes staying in the
 // last-level cache (62).
+// The other form also leaves the workgroup's part of x.y and x.r in part: a dot
+// of two vectors that pass by here anyway, at no pass of its own.
 template <bool RESID>
-__global__ __launch_bounds__(kB) void k_lattice_product(int nf, const double *__restrict__ fst,
+__global__ __launch_bounds__(kB, 5) void k_lattice_product(int nf, const double *__restrict__ fst,
                                                         const int *__restrict__ asym, const double *__restrict__ x,
-                                                        const double *__restrict__ r, double *__restrict__ y) {
+                                                        const double *__restrict__ r, double *__restrict__ y,
+                                                        double *__restrict__ part) {
   const int tot = nf * nf * nf, nblk = (tot + kB - 1) / kB, per = (nblk + 7) / 8;
   const int blk = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
   const int i = blk * kB + threadIdx.x;
-  if (i >= tot) return;
+  if (blk >= nblk) return;
   const int a = i % nf, b = (i / nf) % nf, c = i / (nf * nf);
-  if (a == 0 || b == 0 || c == 0 || a == nf - 1 || b == nf - 1 || c == nf - 1) {
-    y[i] = 0.0;
-    return;
-  }
-  const bool sym = __builtin_amdgcn_readfirstlane(*asym) == 0;
-  double up[13], lo[13], xu[13], xl[13];
+  const bool in = i < tot && a > 0 && b > 0 && c > 0 && a < nf - 1 && b < nf - 1 && c < nf - 1;
+  double acc = 0.0, xi = 0.0, ri = 0.0;
+  if (in) {
+    const bool sym = __builtin_amdgcn_readfirstlane(*asym) == 0;
+    double up[13], lo[13], xu[13], xl[13];
 #pragma unroll
-  for (int k = 0; k < 13; ++k) {
-    const int s = 14 + k, o = slot_offset(s, nf);
-    up[k] = fst[(size_t)s * tot + i];
-    lo[k] = (fst + (sym ? (int64_t)s * tot - o : (int64_t)(26 - s) * tot))[i];
-    xu[k] = x[i + o];
-    xl[k] = x[i - o];
-  }
-  double acc = fst[(size_t)13 * tot + i] * x[i];
+    for (int k = 0; k < 13; ++k) {
+      const int s = 14 + k, o = slot_offset(s, nf);
+      up[k] = fst[(size_t)s * tot + i];
+      lo[k] = (fst + (sym ? (int64_t)s * tot - o : (int64_t)(26 - s) * tot))[i];
+      xu[k] = x[i + o];
+      xl[k] = x[i - o];
+    }
+    xi = x[i];
+    ri = r[i];
+    acc = fst[(size_t)13 * tot + i] * xi;
 #pragma unroll
-  for (int k = 0; k < 13; ++k) acc = fma(up[k], xu[k], fma(lo[k], xl[k], acc));
-  y[i] = RESID ? r[i] - acc : acc;
+    for (int k = 0; k < 13; ++k) acc = fma(up[k], xu[k], fma(lo[k], xl[k], acc));
+  }
+  if (i < tot) y[i] = RESID ? ri - acc : acc;
+  if (!RESID) block_dots(xi * acc, xi * ri, blk, nblk, part);
 }
 
-void lattice_product(TwoGrid *T, const double *x, const double *r, double *y, hipStream_t st) {
-  const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
-  const dim3 g(8 * ((nb(nfl) + 7) / 8)), b(kB);
-  if (r) hipLaunchKernelGGL(k_lattice_product<true>, g, b, 0, st, T->nf, T->fst, T->asym, x, r, y);
-  else hipLaunchKernelGGL(k_lattice_product<false>, g, b, 0, st, T->nf, T->fst, T->asym, x, nullptr, y);
+// sums of both halves of the partials, in a fixed order: into out[0..2), or for
+// alpha their ratio out[0] = second / first (0 when the first vanishes or the
+// ratio is not finite)
+template <bool ALPHA>
+__global__ __launch_bounds__(1024) void k_sum2(const double *__restrict__ part, int nblk, double *__restrict__ out) {
+  __shared__ double s1[1024], s2[1024];
+  const int t = threadIdx.x;
+  double p1 = 0.0, p2 = 0.0;
+  for (int i = t; i < nblk; i += 1024) {
+    p1 += part[i];
+    p2 += part[nblk + i];
+  }
+  s1[t] = p1;
+  s2[t] = p2;
+  __syncthreads();
+  for (int o = 512; o > 0; o >>= 1) {
+    if (t < o) {
+      s1[t] += s1[t + o];
+      s2[t] += s2[t + o];
+    }
+    __syncthreads();
+  }
+  if (t != 0) return;
+  if (ALPHA) {
+    const double al = s2[0] / s1[0];
+    out[0] = s1[0] > 0.0 && isfinite(al) ? al : 0.0;
+  } else {
+    out[0] = s1[0];
+    out[1] = s2[0];
+  }
+}
+
+// x += alpha p, r -= alpha q, alpha = p.r / p.q, and z = w D^-1 r, the first sweep
+__global__ __launch_bounds__(kB) void k_lattice_update(int n, double w, const double *__restrict__ sc,
+                                                       const double *__restrict__ dinv, const double *__restrict__ p,
+                                                       const double *__restrict__ q, double *__restrict__ x,
+                                                       double *__restrict__ r, double *__restrict__ z) {
+  const int i = blockIdx.x * kB + threadIdx.x;
+  if (i >= n) return;
+  const double alpha = sc[1] / sc[0], ri = fma(-alpha, q[i], r[i]);
+  x[i] = fma(alpha, p[i], x[i]);
+  r[i] = ri;
+  z[i] = w * dinv[i] * ri;
+}
+
+// k_coarse_post, with the workgroup's part of z.q and r.r
+__global__ __launch_bounds__(kB) void k_lattice_post(int n, double w, const double *__restrict__ alpha,
+                                                     const double *__restrict__ dinv, const double *__restrict__ s,
+                                                     const double *__restrict__ c, const double *__restrict__ ac,
+                                                     const double *__restrict__ q, const double *__restrict__ r,
+                                                     double *__restrict__ z, double *__restrict__ part) {
+  const int i = blockIdx.x * kB + threadIdx.x;
+  double zi = 0.0, qi = 0.0, ri = 0.0;
+  if (i < n) {
+    const double a = *alpha;
+    zi = fma(a, c[i], z[i]) + w * dinv[i] * fma(-a, ac[i], s[i]);
+    qi = q[i];
+    ri = r[i];
+    z[i] = zi;
+  }
+  block_dots(zi * qi, ri * ri, blockIdx.x, gridDim.x, part);
+}
+
+__global__ void k_lattice_dir(int n, const double *__restrict__ sc, const double *__restrict__ z,
+                              double *__restrict__ p) {
+  const int i = blockIdx.x * kB + threadIdx.x;
+  if (i < n) p[i] = fma(-sc[2] / sc[0], p[i], z[i]);
 }
 
 // network input from a fine residual in global-id order, or on the lattice (s
@@ -1383,45 +1474,87 @@ int twogrid_apply(void *ctx, const double *r, double *z, hipStream_t st) {
 // lattice vectors in T->lat
 enum { kLx, kLr, kLz, kLp, kLq, kLt1, kLt2, kLt3, kLdinv, kLcount };
 
-static int lattice_begin(void *ctx, const double *r, bool current, int *n, double *vecs[5], hipStream_t st) {
-  TwoGrid *T = tg_of(reinterpret_cast<gdx_nn *>(ctx));
-  const int64_t nfl = (int64_t)T->nf * T->nf * T->nf;
+struct LatticeView {
+  gdx_nn *nn;
+  TwoGrid *T;
+  int n, nblk;
+  double *v[kLcount], *part;
+};
+
+static LatticeView lattice_view(void *ctx) {
+  LatticeView L{};
+  L.nn = reinterpret_cast<gdx_nn *>(ctx);
+  L.T = tg_of(L.nn);
+  if (!L.T || !L.T->lat) return L;
+  L.n = L.T->nf * L.T->nf * L.T->nf;
+  L.nblk = (int)nb(L.n);
+  for (int k = 0; k < kLcount; ++k) L.v[k] = L.T->lat + (size_t)k * L.n;
+  L.part = L.T->lat + (size_t)kLcount * L.n;
+  return L;
+}
+
+static int lattice_begin(void *ctx, const double *r, bool current, hipStream_t st) {
+  const LatticeView L = lattice_view(ctx);
+  if (!L.n) return GDX_ERR_STATE;
+  TwoGrid *T = L.T;
+  const size_t bytes = (size_t)L.n * sizeof(double);
   if (!current)
     if (int rc = fine_stencil(T, st)) return rc;
-  // boundary nodes zero: r's and D^-1's here, x's by the solver, and with them every other vector's
+  // boundary nodes zero: x's, r's and D^-1's here, and with them every other vector's
   if (hipMemsetAsync(T->asym, 0, sizeof(int), st) != hipSuccess ||
-      hipMemsetAsync(T->lat + kLr * nfl, 0, nfl * sizeof(double), st) != hipSuccess ||
-      hipMemsetAsync(T->lat + kLdinv * nfl, 0, nfl * sizeof(double), st) != hipSuccess)
+      hipMemsetAsync(L.v[kLx], 0, bytes, st) != hipSuccess || hipMemsetAsync(L.v[kLr], 0, bytes, st) != hipSuccess ||
+      hipMemsetAsync(L.v[kLdinv], 0, bytes, st) != hipSuccess)
     return GDX_ERR_HIP;
-  hipLaunchKernelGGL(k_asymmetric, dim3(nb(nfl)), dim3(kB), 0, st, T->nf, T->fst, T->asym);
-  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, T->dinv, T->lat + kLdinv * nfl);
-  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, T->lat + kLr * nfl);
-  for (int k = 0; k < 5; ++k) vecs[k] = T->lat + k * nfl;
-  *n = (int)nfl;
+  hipLaunchKernelGGL(k_asymmetric, dim3(L.nblk), dim3(kB), 0, st, T->nf, T->fst, T->asym);
+  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, T->dinv, L.v[kLdinv]);
+  hipLaunchKernelGGL(k_scatter, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, r, L.v[kLr]);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-static void lattice_mul(void *ctx, const double *x, double *y, hipStream_t st) {
-  lattice_product(tg_of(reinterpret_cast<gdx_nn *>(ctx)), x, nullptr, y, st);
-}
-
-static int lattice_apply(void *ctx, const double *r, double *z, hipStream_t st) {
-  gdx_nn *nn = reinterpret_cast<gdx_nn *>(ctx);
-  TwoGrid *T = tg_of(nn);
-  const int nfl = T->nf * T->nf * T->nf;
-  double *t1 = T->lat + (size_t)kLt1 * nfl, *t2 = T->lat + (size_t)kLt2 * nfl, *t3 = T->lat + (size_t)kLt3 * nfl;
-  const double *dinv = T->lat + (size_t)kLdinv * nfl;
-  hipLaunchKernelGGL(k_jacobi0, dim3(nb(nfl)), dim3(kB), 0, st, nfl, kOmega, dinv, r, z);
-  lattice_product(T, z, r, t1, st);
-  if (int rc = coarse_correction(nn, T, t1, true, t2, st)) return rc;
-  lattice_product(T, t2, nullptr, t3, st);
-  coarse_step(T, nfl, dinv, t1, t2, t3, z, st);
+// z = M r after z = w D^-1 r, with the partials of z.q and r.r
+static int lattice_precondition(const LatticeView &L, hipStream_t st) {
+  TwoGrid *T = L.T;
+  double *t1 = L.v[kLt1], *t2 = L.v[kLt2], *t3 = L.v[kLt3], *alpha = T->red + kS + 5;
+  const dim3 gp(8 * ((L.nblk + 7) / 8)), g(L.nblk), b(kB);
+  hipLaunchKernelGGL(k_lattice_product<true>, gp, b, 0, st, T->nf, T->fst, T->asym, L.v[kLz], L.v[kLr], t1, nullptr);
+  if (int rc = coarse_correction(L.nn, T, t1, true, t2, st)) return rc;
+  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, T->fst, T->asym, t2, t1, t3, L.part);
+  hipLaunchKernelGGL(k_sum2<true>, dim3(1), dim3(1024), 0, st, L.part, L.nblk, alpha);
+  hipLaunchKernelGGL(k_lattice_post, g, b, 0, st, L.n, kOmega, alpha, L.v[kLdinv], t1, t2, t3, L.v[kLq], L.v[kLr],
+                     L.v[kLz], L.part);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-static void lattice_end(void *ctx, const double *xl, double *x, hipStream_t st) {
-  TwoGrid *T = tg_of(reinterpret_cast<gdx_nn *>(ctx));
-  hipLaunchKernelGGL(k_gather, dim3(nb(T->ng)), dim3(kB), 0, st, T->ng, T->gid_node, xl, x);
+static int lattice_first(void *ctx, hipStream_t st) {
+  const LatticeView L = lattice_view(ctx);
+  if (!L.n) return GDX_ERR_STATE;
+  hipLaunchKernelGGL(k_jacobi0, dim3(L.nblk), dim3(kB), 0, st, L.n, kOmega, L.v[kLdinv], L.v[kLr], L.v[kLz]);
+  if (hipMemsetAsync(L.v[kLq], 0, (size_t)L.n * sizeof(double), st) != hipSuccess) return GDX_ERR_HIP;
+  if (int rc = lattice_precondition(L, st)) return rc;
+  return hipMemcpyAsync(L.v[kLp], L.v[kLz], (size_t)L.n * sizeof(double), hipMemcpyDeviceToDevice, st) == hipSuccess
+             ? GDX_OK
+             : GDX_ERR_HIP;
+}
+
+static int lattice_iterate(void *ctx, double *sc, hipStream_t st) {
+  const LatticeView L = lattice_view(ctx);
+  if (!L.n) return GDX_ERR_STATE;
+  TwoGrid *T = L.T;
+  const dim3 gp(8 * ((L.nblk + 7) / 8)), g(L.nblk), b(kB);
+  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, T->fst, T->asym, L.v[kLp], L.v[kLr], L.v[kLq],
+                     L.part);
+  hipLaunchKernelGGL(k_sum2<false>, dim3(1), dim3(1024), 0, st, L.part, L.nblk, sc);
+  hipLaunchKernelGGL(k_lattice_update, g, b, 0, st, L.n, kOmega, sc, L.v[kLdinv], L.v[kLp], L.v[kLq], L.v[kLx],
+                     L.v[kLr], L.v[kLz]);
+  if (int rc = lattice_precondition(L, st)) return rc;
+  hipLaunchKernelGGL(k_sum2<false>, dim3(1), dim3(1024), 0, st, L.part, L.nblk, sc + 2);
+  hipLaunchKernelGGL(k_lattice_dir, g, b, 0, st, L.n, sc, L.v[kLz], L.v[kLp]);
+  return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+static void lattice_end(void *ctx, double *x, hipStream_t st) {
+  const LatticeView L = lattice_view(ctx);
+  hipLaunchKernelGGL(k_gather, dim3(nb(L.T->ng)), dim3(kB), 0, st, L.T->ng, L.T->gid_node, L.v[kLx], x);
 }
 
 FpcgPrec twogrid_prec(gdx_nn *nn, bool current) {
@@ -1431,15 +1564,16 @@ FpcgPrec twogrid_prec(gdx_nn *nn, bool current) {
   TwoGrid *T = tg_of(nn);
   const int64_t nfl = T ? (int64_t)T->nf * T->nf * T->nf : 0;
   if (!T || nfl >= (int64_t)1 << 30) return p;  // 32-bit node ids in the kernels
-  if (!T->lat && hipMalloc(reinterpret_cast<void **>(&T->lat), (kLcount * nfl + 1) * sizeof(double)) != hipSuccess) {
+  if (!T->lat && hipMalloc(reinterpret_cast<void **>(&T->lat), (kLcount * nfl + 2 * nb(nfl) + 1) * sizeof(double)) !=
+                     hipSuccess) {
     (void)hipGetLastError();
     T->lat = nullptr;  // no room: the products from the CSR rows, in global-id order
   }
   if (T->lat) {
-    T->asym = reinterpret_cast<int *>(T->lat + kLcount * nfl);
+    T->asym = reinterpret_cast<int *>(T->lat + kLcount * nfl + 2 * nb(nfl));
     p.begin = lattice_begin;
-    p.product = lattice_mul;
-    p.apply_lattice = lattice_apply;
+    p.first = lattice_first;
+    p.iterate = lattice_iterate;
     p.end = lattice_end;
     p.current = current;
   }
