@@ -1030,16 +1030,17 @@ __device__ __forceinline__ void block_dots(double a, double b, int blk, int nblk
 // nodes).  The bound is the planes' bytes: 14 x 8 per node against 10 x 27 + 28
 // for the CSR product with 16-bit column codes, and no gather through ids.
 // 128^3 cells: 80 us (the CSR product 144); 96^3: 25 us, its planes staying in the
-// last-level cache (62).
+// last-level cache (62).  back walks the nodes from their end: after a product in
+// the other direction the planes read last are still in that cache (70 us).
 // The other form also leaves the workgroup's part of x.y and x.r in part: a dot
 // of two vectors that pass by here anyway, at no pass of its own.
 template <bool RESID>
-__global__ __launch_bounds__(kB, 5) void k_lattice_product(int nf, const double *__restrict__ fst,
+__global__ __launch_bounds__(kB, 5) void k_lattice_product(int nf, int back, const double *__restrict__ fst,
                                                         const int *__restrict__ asym, const double *__restrict__ x,
                                                         const double *__restrict__ r, double *__restrict__ y,
                                                         double *__restrict__ part) {
   const int tot = nf * nf * nf, nblk = (tot + kB - 1) / kB, per = (nblk + 7) / 8;
-  const int blk = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int at = (int)(blockIdx.x / 8), blk = (int)(blockIdx.x % 8) * per + (back ? per - 1 - at : at);
   const int i = blk * kB + threadIdx.x;
   if (blk >= nblk) return;
   const int a = i % nf, b = (i / nf) % nf, c = i / (nf * nf);
@@ -1516,9 +1517,9 @@ static int lattice_precondition(const LatticeView &L, hipStream_t st) {
   TwoGrid *T = L.T;
   double *t1 = L.v[kLt1], *t2 = L.v[kLt2], *t3 = L.v[kLt3], *alpha = T->red + kS + 5;
   const dim3 gp(8 * ((L.nblk + 7) / 8)), g(L.nblk), b(kB);
-  hipLaunchKernelGGL(k_lattice_product<true>, gp, b, 0, st, T->nf, T->fst, T->asym, L.v[kLz], L.v[kLr], t1, nullptr);
+  hipLaunchKernelGGL(k_lattice_product<true>, gp, b, 0, st, T->nf, 1, T->fst, T->asym, L.v[kLz], L.v[kLr], t1, nullptr);
   if (int rc = coarse_correction(L.nn, T, t1, true, t2, st)) return rc;
-  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, T->fst, T->asym, t2, t1, t3, L.part);
+  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, 0, T->fst, T->asym, t2, t1, t3, L.part);
   hipLaunchKernelGGL(k_sum2<true>, dim3(1), dim3(1024), 0, st, L.part, L.nblk, alpha);
   hipLaunchKernelGGL(k_lattice_post, g, b, 0, st, L.n, kOmega, alpha, L.v[kLdinv], t1, t2, t3, L.v[kLq], L.v[kLr],
                      L.v[kLz], L.part);
@@ -1541,7 +1542,7 @@ static int lattice_iterate(void *ctx, double *sc, hipStream_t st) {
   if (!L.n) return GDX_ERR_STATE;
   TwoGrid *T = L.T;
   const dim3 gp(8 * ((L.nblk + 7) / 8)), g(L.nblk), b(kB);
-  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, T->fst, T->asym, L.v[kLp], L.v[kLr], L.v[kLq],
+  hipLaunchKernelGGL(k_lattice_product<false>, gp, b, 0, st, T->nf, 0, T->fst, T->asym, L.v[kLp], L.v[kLr], L.v[kLq],
                      L.part);
   hipLaunchKernelGGL(k_sum2<false>, dim3(1), dim3(1024), 0, st, L.part, L.nblk, sc);
   hipLaunchKernelGGL(k_lattice_update, g, b, 0, st, L.n, kOmega, sc, L.v[kLdinv], L.v[kLp], L.v[kLq], L.v[kLx],
