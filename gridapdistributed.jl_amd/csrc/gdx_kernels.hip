@@ -69,12 +69,20 @@ __global__ void k_fourier_tables(const double *__restrict__ modes, KParams kp, i
 // in registers across the lines; the per-line (y,z) products b = e2 e3 and
 // (k.c) b are tabulated in LDS, so each (point, mode) costs four FMAs:
 //   g += Re(e1 b),  s += Im(e1 (k.c) b).
-constexpr int kCoefLines = 8, kCoefModes = 16;
+//
+// A wave reads two (four) of the tabulated doubles from LDS for every two (four)
+// FMAs, and four SIMDs share that LDS port: the reads bound it (7.1 M points, 16
+// modes, both sums: 48 us, at 128 B per clock and CU the reads alone 46).  So a
+// problem whose source is constant makes the first sum only and stores no f
+// where no kernel reads one (SOURCE = false), and up to 8 modes go in a chunk of
+// 8: 32 Q1 cubes of 16..48 cells with 8 modes 97 -> 43 us.
+constexpr int kCoefLines = 8;
 
+template <bool SOURCE, int MODES>
 __device__ __forceinline__ void coefficient_lines(const double *__restrict__ modes, const double *__restrict__ E,
                                                   const KParams &kp, int qnmax, double *__restrict__ W,
                                                   double *__restrict__ F, int bx, int by, int q3) {
-  __shared__ double tb[kCoefLines][kCoefModes][4];  // br, bi, (k.c) br, (k.c) bi
+  __shared__ double tb[kCoefLines][MODES][SOURCE ? 4 : 2];  // br, bi, (k.c) br, (k.c) bi
   const int q1 = bx * blockDim.x + threadIdx.x;
   const int q2b = by * kCoefLines;
   const bool active = q1 < kp.qn[0];
@@ -82,10 +90,10 @@ __device__ __forceinline__ void coefficient_lines(const double *__restrict__ mod
   double g[kCoefLines], s[kCoefLines];
 #pragma unroll
   for (int l = 0; l < kCoefLines; ++l) g[l] = s[l] = 0.0;
-  for (int m0 = 0; m0 < nm; m0 += kCoefModes) {
+  for (int m0 = 0; m0 < nm; m0 += MODES) {
     __syncthreads();
-    for (int i = threadIdx.x; i < kCoefLines * kCoefModes; i += blockDim.x) {
-      const int l = i / kCoefModes, j = i % kCoefModes, m = m0 + j;
+    for (int i = threadIdx.x; i < kCoefLines * MODES; i += blockDim.x) {
+      const int l = i / MODES, j = i % MODES, m = m0 + j;
       const int q2 = q2b + l < kp.qn[1] ? q2b + l : kp.qn[1] - 1;
       double br = 0.0, bi = 0.0, kc = 0.0;
       if (m < nm) {
@@ -98,13 +106,15 @@ __device__ __forceinline__ void coefficient_lines(const double *__restrict__ mod
       }
       tb[l][j][0] = br;
       tb[l][j][1] = bi;
-      tb[l][j][2] = kc * br;
-      tb[l][j][3] = kc * bi;
+      if constexpr (SOURCE) {
+        tb[l][j][2] = kc * br;
+        tb[l][j][3] = kc * bi;
+      }
     }
     __syncthreads();
-    double e1r[kCoefModes], e1i[kCoefModes];
+    double e1r[MODES], e1i[MODES];
 #pragma unroll
-    for (int j = 0; j < kCoefModes; ++j) {
+    for (int j = 0; j < MODES; ++j) {
       const bool ok = active && m0 + j < nm;
       const double *e1 = E + 2 * ((size_t)(ok ? m0 + j : 0) * qnmax + (active ? q1 : 0));
       e1r[j] = ok ? e1[0] : 0.0;
@@ -113,9 +123,9 @@ __device__ __forceinline__ void coefficient_lines(const double *__restrict__ mod
 #pragma unroll
     for (int l = 0; l < kCoefLines; ++l) {
 #pragma unroll
-      for (int j = 0; j < kCoefModes; ++j) {
+      for (int j = 0; j < MODES; ++j) {
         g[l] = fma(e1r[j], tb[l][j][0], fma(-e1i[j], tb[l][j][1], g[l]));
-        s[l] = fma(e1r[j], tb[l][j][3], fma(e1i[j], tb[l][j][2], s[l]));
+        if constexpr (SOURCE) s[l] = fma(e1r[j], tb[l][j][3], fma(e1i[j], tb[l][j][2], s[l]));
       }
     }
   }
@@ -128,14 +138,15 @@ __device__ __forceinline__ void coefficient_lines(const double *__restrict__ mod
     const size_t idx = q1 + (size_t)kp.qn[0] * (q2 + (size_t)kp.qn[1] * q3);
     W[idx] = kap;
     // f = -div(kappa grad uD) = -kappa grad(g).c = kappa 2 pi sum_m (k_m.c) a_m sin(theta_m)
-    F[idx] = kp.rhs_kind == GDX_RHS_MANUFACTURED ? kap * 2.0 * M_PI * s[l] : kp.rhs_const;
+    if (F) F[idx] = SOURCE && kp.rhs_kind == GDX_RHS_MANUFACTURED ? kap * 2.0 * M_PI * s[l] : kp.rhs_const;
   }
 }
 
+template <bool SOURCE, int MODES>
 __global__ __launch_bounds__(256) void k_coefficients(const double *__restrict__ modes,
                                                       const double *__restrict__ E, KParams kp, int qnmax,
                                                       double *__restrict__ W, double *__restrict__ F) {
-  coefficient_lines(modes, E, kp, qnmax, W, F, blockIdx.x, blockIdx.y, blockIdx.z);
+  coefficient_lines<SOURCE, MODES>(modes, E, kp, qnmax, W, F, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // The same for many problems at once: a block finds its problem and its place
@@ -159,11 +170,12 @@ __global__ __launch_bounds__(256) void k_fourier_tables_batch(const CoefProblem 
   fourier_table(p.modes, p.kp, p.qnmax, p.E, b.y, b.z, threadIdx.x, blockDim.x);
 }
 
+template <bool SOURCE, int MODES>  // what the problem that needs most needs
 __global__ __launch_bounds__(64) void k_coefficients_batch(const CoefProblem *__restrict__ probs,
-                                                            const CoefBlock *__restrict__ blocks) {
+                                                           const CoefBlock *__restrict__ blocks) {
   const CoefBlock b = blocks[blockIdx.x];
   const CoefProblem &p = probs[b.prob];
-  coefficient_lines(p.modes, p.E, p.kp, p.qnmax, p.W, p.F, b.x, b.y, b.z);
+  coefficient_lines<SOURCE, MODES>(p.modes, p.E, p.kp, p.qnmax, p.W, p.F, b.x, b.y, b.z);
 }
 
 // ---------------------------------------------------------------------------
@@ -176,6 +188,12 @@ static int longest_line(const KParams &kp) {
 }
 
 bool points_used(const gdx_problem *p) { return !lattice_used(p) || (!p->coef_cell && p->kp.nmodes > 0); }
+
+// f at the quadrature points, where a kernel reads it: the pair-lattice kernel
+// takes a constant f in closed form
+static double *source_array(const gdx_problem *p) {
+  return lattice_used(p) && p->kp.rhs_kind != GDX_RHS_MANUFACTURED ? nullptr : p->dev.F;
+}
 
 int launch_coefficients(gdx_problem *p, hipStream_t st) {
   // the pair-lattice kernel takes a coefficient that is constant on every cell as it is
@@ -193,7 +211,10 @@ int launch_coefficients(gdx_problem *p, hipStream_t st) {
   }
   const int bx = kp.qn[0] < 256 ? 64 * ((kp.qn[0] + 63) / 64) : 256;
   dim3 g2((kp.qn[0] + bx - 1) / bx, (kp.qn[1] + kCoefLines - 1) / kCoefLines, kp.qn[2]);
-  GDX_LAUNCH(p, k_coefficients, g2, dim3(bx), st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, p->dev.F);
+  const bool source = kp.rhs_kind == GDX_RHS_MANUFACTURED, few = kp.nmodes <= 8;
+  const auto kernel = source ? (few ? k_coefficients<true, 8> : k_coefficients<true, 16>)
+                             : (few ? k_coefficients<false, 8> : k_coefficients<false, 16>);
+  GDX_LAUNCH(p, kernel, g2, dim3(bx), st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, source_array(p));
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
@@ -204,6 +225,7 @@ struct CoefBatch {
   CoefProblem *probs = nullptr;
   CoefBlock *tables = nullptr, *lines = nullptr;
   unsigned ntables = 0, nlines = 0;
+  bool source = false, few = true;
 };
 
 void coef_batch_free(CoefBatch *b) {
@@ -221,7 +243,7 @@ int coef_batch_build(const std::vector<gdx_problem *> &ps, CoefBatch **out) {
   for (gdx_problem *p : ps) {
     const KParams &kp = p->kp;
     const int i = (int)probs.size();
-    probs.push_back({kp, p->dev.modes, p->dev.E, p->dev.W, p->dev.F, longest_line(kp)});
+    probs.push_back({kp, p->dev.modes, p->dev.E, p->dev.W, source_array(p), longest_line(kp)});
     for (int d = 0; d < 3; ++d)
       for (int m = 0; m < kp.nmodes; ++m) tables.push_back({i, 0, m, d});
     for (int z = 0; z < kp.qn[2]; ++z)
@@ -241,13 +263,19 @@ int coef_batch_build(const std::vector<gdx_problem *> &ps, CoefBatch **out) {
   }
   b->ntables = (unsigned)tables.size();
   b->nlines = (unsigned)lines.size();
+  for (gdx_problem *p : ps) {
+    b->source |= p->kp.rhs_kind == GDX_RHS_MANUFACTURED;
+    b->few &= p->kp.nmodes <= 8;
+  }
   *out = b;
   return GDX_OK;
 }
 
 int coef_batch_launch(const CoefBatch *b, hipStream_t st) {
   if (b->ntables) hipLaunchKernelGGL(k_fourier_tables_batch, dim3(b->ntables), dim3(256), 0, st, b->probs, b->tables);
-  if (b->nlines) hipLaunchKernelGGL(k_coefficients_batch, dim3(b->nlines), dim3(64), 0, st, b->probs, b->lines);
+  const auto lines = b->source ? (b->few ? k_coefficients_batch<true, 8> : k_coefficients_batch<true, 16>)
+                               : (b->few ? k_coefficients_batch<false, 8> : k_coefficients_batch<false, 16>);
+  if (b->nlines) hipLaunchKernelGGL(lines, dim3(b->nlines), dim3(64), 0, st, b->probs, b->lines);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 

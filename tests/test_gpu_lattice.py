@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from _helpers import STRUCT_KEYS, rel_err
-from gridap_amd import problem_from_workload
+from gridap_amd import AssemblyBatch, problem_from_workload
 from gridap_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +77,62 @@ def test_lattice_kernel_matches_oracle(gpu_ctx, p):
         if len(P["b"]):
             assert np.abs(Q["b"] - P["b"]).max() <= 1e-12 * max(np.abs(P["b"]).max(), np.abs(P["val"]).max())
     prob.close()
+
+
+def check(r, prob):
+    for k, P in enumerate(r.parts):
+        Q = prob.export_part(k)
+        if len(P["val"]):
+            assert rel_err(Q["val"], P["val"]) <= 1e-12, k
+        if len(P["b"]):
+            assert np.abs(Q["b"] - P["b"]).max() <= 1e-12 * max(np.abs(P["b"]).max(), np.abs(P["val"]).max()), k
+
+
+# chunks of 8 (up to 8 modes) and of 16, whole and ragged, with and without the source's sum; lines of 64 points and more
+@pytest.mark.parametrize("nmodes", [1, 8, 9, 16, 17])
+@pytest.mark.parametrize("rhs", ["const", "manufactured"])
+def test_coefficient_mode_chunks_match_oracle(gpu_ctx, nmodes, rhs):
+    p = dict(case((33, 4, 3), (2, 1, 1), 1, "points"), rhs=rhs)
+    p["modes"] = W.fourier_modes(nmodes, nmodes, 3, 0.4)
+    r = oracle.run(p)
+    assem, data = problem_from_workload(gpu_ctx, p)
+    prob = assem._problem_for(data)
+    # and the other kernels, which read f at the points also where it is constant
+    for variant in (2, 1, 2, 0):
+        prob.set_kernel(variant)
+        prob.numeric()
+        prob.sync()
+        check(r, prob)
+    prob.close()
+
+
+@pytest.mark.parametrize("few", [True, False], ids=["up to 8 modes", "more"])
+@pytest.mark.parametrize("source", [False, True], ids=["f constant", "f varies"])
+def test_mixed_batch_matches_oracle(gpu_ctx, few, source):
+    """Every tile shape and form of the coefficient in one batch, with a problem
+    that no pair lattice takes beside them."""
+    ps = [case((6, 5, 4), (2, 1, 1), 1, "points"), case((5, 4, 3), (1, 2, 1), 2, "points"),
+          case((17, 9), (2, 1), 1, "points"), case((9, 8), (1, 1), 2, "points"), case((16, 8, 4), (1, 1, 1), 1, "const"),
+          case((4, 3, 3), (1, 1, 1), 2, "const"), case((7, 7, 5), (1, 1, 2), 1, "const")]
+    if not few:
+        ps[0]["modes"] = W.fourier_modes(12, 12, 3, 0.4)
+    if source:
+        ps[1]["rhs"] = "manufactured"
+        ps[2]["rhs"] = "manufactured"
+    refs, probs = [oracle.run(p) for p in ps], []
+    b = AssemblyBatch(gpu_ctx)
+    for k, p in enumerate(ps):
+        assem, data = problem_from_workload(gpu_ctx, p)
+        probs.append(assem._problem_for(data))
+        b.add(probs[-1])
+    b.autotune(1)
+    probs[-1].set_kernel(1)
+    b.capture()
+    for _ in range(3):
+        b.launch()
+        b.sync()
+        for r, prob in zip(refs, probs):
+            check(r, prob)
+    b.close()
+    for prob in probs:
+        prob.close()
