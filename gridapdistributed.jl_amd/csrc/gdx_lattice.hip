@@ -21,9 +21,9 @@
 // points first, which is the same quadrature.
 //
 // Measured against the z-marching kernel that was the default before, whole
-// numeric phases: 3D Q2 64^3, Fourier kappa 0.86 -> 0.52 ms (the matrix kernel
-// 790 -> 420 us); 3D Q1 131 x 97 x 75, kappa per cell 517 -> 85 us (453 -> 50);
-// 2D Q1 256^2 95 -> 28 us (71 -> 9).  The Q2 kernel writes 2.4 TB/s of the 6.7
+// numeric phases: 3D Q2 64^3, Fourier kappa 0.86 -> 0.51 ms (the matrix kernel
+// 790 -> 410 us); 3D Q1 131 x 97 x 75, kappa per cell 517 -> 70 us (453 -> 50);
+// 2D Q1 256^2 95 -> 18 us (71 -> 9).  The Q2 kernel writes 2.4 TB/s of the 6.7
 // that a fill reaches; what is left is latency: at two workgroups per CU the
 // LDS contraction (about 40% of a tile's time) hides behind little else.
 //
@@ -867,7 +867,8 @@ int launch_lattice(gdx_problem *p, hipStream_t st) {
 
 // Tiles of many problems, one launch per instance.  A small problem's own launch
 // fills a few CUs: 32 Q1 cubes of 16..48 cells on four branches of a graph took
-// 0.65 ms, the single launch (with the coefficients' two) 0.2 ms.
+// 0.87 ms a refill, the single launch (with the coefficients' two) 0.30 ms, 0.18 of
+// them in this kernel.
 struct LatticeBatch {
   LatArgs *probs = nullptr;
   struct Group {

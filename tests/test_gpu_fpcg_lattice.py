@@ -11,7 +11,8 @@ import pytest
 import scipy.sparse as sp
 import scipy.sparse.linalg as spl
 
-from coarse_bound import Multilevel
+import nn_oracle as NO
+from coarse_bound import Multilevel, prolong3
 from gridap_amd import LearnedCoarseSolver, _lib, fpcg, problem_from_workload
 from gridap_amd import workloads as W
 
@@ -101,5 +102,64 @@ def test_vcycle_matches_reference(gpu_ctx, n, nu):
     zr = ref(r[order])
     # rounding of 27 products a sweep, about 100 sweeps deep (1e-12), times the spread of the diagonals (about 1e2)
     assert np.linalg.norm(z - zr) <= 1e-10 * np.linalg.norm(zr)
+    net.close()
+    prob.close()
+
+
+def mix64(z):
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
+
+
+def means(e, passes):
+    """3x3x3 means over the interior nodes, zero outside"""
+    for _ in range(passes):
+        p = np.pad(e, 1)
+        e = sum(p[k : k + e.shape[0], j : j + e.shape[1], i : i + e.shape[2]]
+                for k in range(3) for j in range(3) for i in range(3)) / 27.0
+    return e
+
+
+# three means a launch and one or two in the last; 8 and 20 nodes: less than a 16 x 8 x 8 tile, and tiles cut short
+@pytest.mark.parametrize("n", [8, 20])
+def test_training_sample_matches_reference(gpu_ctx, n):
+    assem, data = problem_from_workload(gpu_ctx, W.poisson3d_q1(2 * n, (1, 1, 1), rhs_const=0.0))
+    prob = assem._problem_for(data)
+    prob.cell_coefficient_grf(9, 0.1, 2.0)
+    prob.numeric()
+    prob.sync()
+    P = prob.export_part(0)
+    order = P["ldof_gid"][np.argsort(P["ldof_gnode"])] - P["ldof_gid"].min()
+    A = matrix(prob, 1).tocsr()[order][:, order]
+    net = LearnedCoarseSolver(gpu_ctx, n, 1)
+    theta = net.get_params()
+    Pr, dinv, m, seed = prolong3(2 * n), 1.0 / A.diagonal(), n - 1, 77
+    z, y, x = np.meshgrid(*[np.arange(m, dtype=np.uint64)] * 3, indexing="ij")
+    j = x + np.uint64(n) * (y + np.uint64(n) * z)
+    with np.errstate(over="ignore"):
+        h = mix64(np.uint64(seed) * np.uint64(0x9E3779B97F4A7C15) + (j + np.uint64(1)) * np.uint64(0xD1B54A32D192ED03))
+    noise = 2.0 * (((h >> np.uint64(11)).astype(np.float64) + 0.5) / 2.0**53) - 1.0
+    dcoarse = dinv.reshape((2 * n - 1,) * 3)[1::2, 1::2, 1::2]
+    ref = []
+    for passes in range(9):
+        ec = means(noise, passes)
+        rho = (Pr.T @ (A @ (Pr @ ec.ravel().astype(np.float32).astype(np.float64)))).reshape(ec.shape) * dcoarse
+        inp = np.zeros((2, n, n, n), np.float32)
+        s = np.sqrt((rho**2).sum() / n**3)
+        inp[0, :m, :m, :m] = rho / s
+        inp[1, :m, :m, :m] = 0.5 * (-np.log(dcoarse / (2 * n)) - np.log(8.0 / 3.0))
+        out = NO.forward(inp, theta, (8, 16, 24))[0][0]
+        t = np.zeros((n, n, n))
+        t[:m, :m, :m] = ec / s
+        ref.append(1.0 - (out * t).sum() ** 2 / ((out**2).sum() * (t**2).sum()))
+    # the device's activations differ from the oracle's by single BF16 roundings (2^-9) here and there, far less in a
+    # loss that sums n^3 of them; one mean more or less moves it by more than that
+    tol = 1e-4
+    assert np.abs(np.diff(ref)).min() > 2 * tol
+    for passes in range(9):
+        net.set_params(theta)
+        net.attach(prob)
+        assert abs(net.train_step(seed, 1e-3, smooth_passes=passes) - ref[passes]) <= tol, passes
     net.close()
     prob.close()
