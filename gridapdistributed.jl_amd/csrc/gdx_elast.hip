@@ -48,6 +48,7 @@
 #include <vector>
 
 #include "gdx_internal.h"
+#include "gdx_launch.h"
 
 namespace gdx {
 

@@ -1,6 +1,5 @@
 // Internal data structures of libgdx (host side).
 #pragma once
-#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -204,17 +203,6 @@ struct gdx_problem {
   void *pv = nullptr;     // PRange maps of the device PVectors (gdx_pvector.hip)
   std::vector<gdx_pvector *> pvecs;  // live PVectors on this problem
 };
-
-// Launch of a numeric phase's kernel.  The phase's events ride on the kernels'
-// own packets: an event record of its own costs a barrier and a cache flush,
-// about 5 us of the stream each.
-#define GDX_LAUNCH(p, kernel, grid, block, st, ...)                                                              \
-  do {                                                                                                           \
-    if ((p)->launch_ev[0] || (p)->launch_ev[1])                                                                  \
-      hipExtLaunchKernelGGL(kernel, grid, block, 0, st, (p)->launch_ev[0], (p)->launch_ev[1], 0, __VA_ARGS__);   \
-    else                                                                                                         \
-      hipLaunchKernelGGL(kernel, grid, block, 0, st, __VA_ARGS__);                                               \
-  } while (0)
 
 namespace gdx {
 void set_error(const std::string &msg);

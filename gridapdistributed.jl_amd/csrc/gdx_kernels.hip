@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "gdx_device.h"
+#include "gdx_launch.h"
 
 namespace gdx {
 

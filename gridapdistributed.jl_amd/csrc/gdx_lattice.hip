@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "gdx_device.h"
+#include "gdx_launch.h"
 #include "gdx_lattice.h"
 
 namespace gdx {

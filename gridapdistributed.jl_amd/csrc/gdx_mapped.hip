@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "gdx_internal.h"
+#include "gdx_launch.h"
 
 namespace gdx {
 
