@@ -816,12 +816,19 @@ int lattice_setup(gdx_problem *p) {
   LatArgs a{};
   geometry(p, a);
   const size_t n = (size_t)a.pn[0] * a.pn[1] * a.pn[2];
-  int *node_part = nullptr;
-  LatPart *dparts = nullptr;
+  // one buffer and one copy: the position tables, then what the row table is made from
+  const auto up16 = [](size_t bytes) { return (bytes + 15) / 16 * 16; };
+  const size_t at_parts = up16(delta.size() * sizeof(uint16_t)), at_np = at_parts + up16(parts.size() * sizeof(LatPart));
+  std::vector<char> tab(at_np + up16(np.size() * sizeof(int)), 0);
+  std::copy_n(reinterpret_cast<const char *>(delta.data()), delta.size() * sizeof(uint16_t), tab.data());
+  std::copy_n(reinterpret_cast<const char *>(parts.data()), parts.size() * sizeof(LatPart), tab.data() + at_parts);
+  std::copy_n(reinterpret_cast<const char *>(np.data()), np.size() * sizeof(int), tab.data() + at_np);
+  char *dtab = nullptr;
   int rc = GDX_OK;
-  if (put(&node_part, np) != hipSuccess || put(&dparts, parts) != hipSuccess || put(&L->delta, delta) != hipSuccess ||
-      dev_malloc(&L->rows, n * sizeof(LatRow)) != hipSuccess)
-    rc = GDX_ERR_ALLOC;
+  if (put(&dtab, tab) != hipSuccess || dev_malloc(&L->rows, n * sizeof(LatRow)) != hipSuccess) rc = GDX_ERR_ALLOC;
+  L->delta = reinterpret_cast<uint16_t *>(dtab);
+  const LatPart *dparts = reinterpret_cast<const LatPart *>(dtab + at_parts);
+  const int *node_part = reinterpret_cast<const int *>(dtab + at_np);
   if (!rc) {
     hipStream_t st = p->ctx->stream;
     const dim3 g((a.pn[0] + 255) / 256, a.pn[1], a.pn[2]);
@@ -830,8 +837,6 @@ int lattice_setup(gdx_problem *p) {
                        p->dev.rowinfo, L->rows);
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) rc = GDX_ERR_HIP;
   }
-  if (node_part) (void)hipFree(node_part);
-  if (dparts) (void)hipFree(dparts);
   if (rc) lattice_free(p);
   return rc;
 }
