@@ -372,8 +372,10 @@ __device__ __forceinline__ void lattice_tile(ArgsRef a, int tile) {
     constexpr int G = 4;
     const int off_lo = (int)row.off, off_hi = (int)(row.off >> 32);
     // Every row is stored through a buffer resource of exactly its length, so
-    // the lanes beyond it need no branch; the offset tables of the next line go
-    // out before this line's stores, which they then never wait for.
+    // the lanes beyond it need no branch (a chunk's offset is part of the vector
+    // offset: the scalar offset does not count in the bounds check); the offset
+    // tables of the next line go out before this line's stores, which they then
+    // never wait for.
     auto lines = [&](int la, int lb, auto chunks) {
       constexpr int CH = decltype(chunks)::value;  // 64-entry chunks of the longest row
       if (la >= lb) return;
@@ -412,7 +414,7 @@ __device__ __forceinline__ void lattice_tile(ArgsRef a, int tile) {
               reinterpret_cast<char *>(a.values) + off, 0, 8 * (mt & 0xFF), 0x00020000);
 #pragma unroll
           for (int c = 0; c < CH; ++c)
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(UInt2, v[g][c]), rs, 8 * lane, 512 * c, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(UInt2, v[g][c]), rs, 8 * lane + 512 * c, 0, 0);
         }
       }
     };

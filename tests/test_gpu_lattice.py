@@ -38,6 +38,8 @@ CASES = [
     # Q2 tiles are 4 x 4 x 2 cells in 3D and 8 x 8 in 2D, Q1 tiles 15 x 7 x 3 (4 for kappa per cell) and 16 x 16 rows
     case((4, 4, 2), (1, 1, 1), 2, "manufactured"), case((5, 3, 3), (2, 1, 1), 2, "manufactured"),
     case((9, 8, 4), (2, 2, 1), 2, "cells"), case((1, 1, 1), (1, 1, 1), 2, "points", dirichlet=False),
+    # thin: every row shorter than one 64-entry chunk; and rows of both chunks in front of ghost rows, which stay zero
+    case((1, 1, 5), (1, 1, 2), 2, "cells", dirichlet=False), case((6, 3, 3), (2, 1, 1), 2, "points", dirichlet=False),
     case((2, 1, 5), (1, 1, 2), 2, "const", dirichlet=False), case((4, 5, 3), (1, 1, 1), 2, "points", strategy="full", qdeg=2),
     case((8, 4, 2), (1, 2, 1), 2, "const-manufactured", dirichlet=False),
     case((16, 8, 4), (1, 1, 1), 1, "manufactured"), case((17, 9, 5), (2, 1, 2), 1, "cells"),
@@ -74,6 +76,7 @@ def test_lattice_kernel_matches_oracle(gpu_ctx, p):
             assert np.array_equal(P[key], Q[key]), (k, key)
         if len(P["val"]):
             assert rel_err(Q["val"], P["val"]) <= 1e-12
+        assert np.all(Q["val"][Q["rowptr"][P["n_own"]]:] == 0.0)
         if len(P["b"]):
             assert np.abs(Q["b"] - P["b"]).max() <= 1e-12 * max(np.abs(P["b"]).max(), np.abs(P["val"]).max())
     prob.close()
