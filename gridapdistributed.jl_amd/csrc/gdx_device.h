@@ -119,7 +119,10 @@ __device__ __forceinline__ double uD_at(const KParams &kp, int g0, int g1, int g
 
 // sum_k val[k] x[col[k]] of one row by LPR lanes: each lane's share, U entries at
 // a time with their values and ids loaded before the first gather (one at a time
-// every entry waited for its id, then for its x).  Values and ids are read once.
+// every entry waited for its id, then for its x).  Ordinary loads: a program
+// multiplies by the same matrix again, and one of up to 256 MB is still in the
+// caches then (nontemporal loads lose that: Q1 96 x 80 x 90 44 us against 73, one
+// entry at a time 60; 128^3, 0.7 GB: 171 against 216, 221).
 template <int LPR, int U>
 __device__ __forceinline__ double row_product(const double *__restrict__ val, const int *__restrict__ col, int len,
                                               int lane, const double *__restrict__ x) {
@@ -130,8 +133,8 @@ __device__ __forceinline__ double row_product(const double *__restrict__ val, co
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool in = k0 + u * LPR < len;
-      c[u] = in ? __builtin_nontemporal_load(col + k0 + u * LPR) : -1;
-      v[u] = in ? __builtin_nontemporal_load(val + k0 + u * LPR) : 0.0;
+      c[u] = in ? col[k0 + u * LPR] : -1;
+      v[u] = in ? val[k0 + u * LPR] : 0.0;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) xv[u] = c[u] >= 0 ? x[c[u]] : 0.0;

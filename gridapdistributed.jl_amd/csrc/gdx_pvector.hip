@@ -249,8 +249,12 @@ int build_mul(gdx_problem *p) {
     cbase += P.ncols;
   }
   // Q2 rows (27..125 entries, 62 on average): 16 lanes keep 94% of their loads in
-  // use, 32 lanes 80%
-  D->lpr = maxlen > 192 ? 32 : (maxlen > 32 ? 16 : 8);
+  // use, 32 lanes 80% (48^3 163 us against 208; elasticity's rows of up to 81 entries,
+  // 64 x 60 x 50 Q1, 133 against 158).  27-entry rows take 8 (Q1 96 x 80 x 90 44 us, 16
+  // lanes 58), 9-entry rows 4, one round of four loads (2D Q1 700 x 650 17 us, 8 lanes
+  // 22), elasticity's Q2 rows of up to 375 take 32 (12 x 13 x 12 22.2 us against 22.9
+  // with 16, 6^3 7.2 against 7.6; at 40 x 36 x 32 539 against 520)
+  D->lpr = maxlen > 192 ? 32 : (maxlen > 32 ? 16 : (maxlen > 16 ? 8 : 4));
   if (!upload(&D->rstart, rstart) || !upload(&D->rlen, rlen) || !upload(&D->rcb, rcb) ||
       !upload(&D->colidx, colidx)) {
     set_error("device allocation failed for the local CSR column ids");
@@ -492,7 +496,9 @@ int gdx_psparse_mul(gdx_problem *p, gdx_pvector *y, gdx_pvector *x) {
   const int64_t n = p->rows_total;
   if (n > 0) {
     const dim3 g((unsigned)((n * D->lpr + gdx::kB - 1) / gdx::kB)), b(gdx::kB);
-    if (D->lpr == 8)
+    if (D->lpr == 4)
+      hipLaunchKernelGGL(gdx::k_pv_mul<4>, g, b, 0, st, n, D->rstart, D->rlen, D->rcb, D->colidx, p->dev.values, x->v, y->v);
+    else if (D->lpr == 8)
       hipLaunchKernelGGL(gdx::k_pv_mul<8>, g, b, 0, st, n, D->rstart, D->rlen, D->rcb, D->colidx, p->dev.values, x->v, y->v);
     else if (D->lpr == 16)
       hipLaunchKernelGGL(gdx::k_pv_mul<16>, g, b, 0, st, n, D->rstart, D->rlen, D->rcb, D->colidx, p->dev.values, x->v, y->v);
