@@ -485,6 +485,7 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
   GDX_HIP(hipSetDevice(p->ctx->device));
   hipStream_t st = p->ctx->stream;
   for (bool &e : p->ev_set) e = false;
+  p->timed = false;
   const bool diffusion = p->desc.op_kind == GDX_OP_DIFFUSION;
   if (p->desc.op_kind == GDX_OP_FLUX || (diffusion && !p->mapped && !gdx::lattice_used(p))) {
     // stages of several kernels: event records between them
@@ -511,7 +512,7 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
       p->ev_set[1] = p->ev_set[2] = true;
     }
     GDX_HIP(hipEventRecord(p->ev[3], st));
-    p->ev_set[0] = p->ev_set[3] = true;
+    p->ev_set[0] = p->ev_set[3] = p->timed = true;
     return GDX_OK;
   }
   // every other stage is timed by its own kernels' packets
@@ -535,10 +536,11 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
     stage(true, 3, [&] { return gdx::launch_matrix(p, st); });
   }
   if (rc) {
-    for (bool &e : p->ev_set) e = false;
     set_error("numeric kernel launch failed");
+    return rc;
   }
-  return rc;
+  p->timed = true;
+  return GDX_OK;
 }
 
 int gdx_problem_set_kernel(gdx_problem *p, int32_t variant, int32_t rows_z) {
@@ -752,6 +754,7 @@ int gdx_phase_times(gdx_problem *p, double *ms, int32_t n) {
   GDX_REQUIRE(p && ms && n >= 0, GDX_ERR_ARG, "NULL argument");
   GDX_REQUIRE(p->symbolic_done, GDX_ERR_STATE, "gdx_symbolic has not run");
   GDX_REQUIRE(p->ctx, GDX_ERR_STATE, "host-only problem (created without a context)");
+  GDX_REQUIRE(p->timed, GDX_ERR_STATE, "no numeric phase has run, or the last one failed");
   float t[4] = {0, 0, 0, 0};
   int last = 0;
   for (int k = 1; k < 4; ++k) {

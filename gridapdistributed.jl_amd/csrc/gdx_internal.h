@@ -187,6 +187,7 @@ struct gdx_problem {
   // coefficient, RHS and matrix stages (ev_set: the stages that launched)
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   bool ev_set[4] = {false, false, false, false};
+  bool timed = false;  // a numeric phase has run (and the last one did not fail)
   // start and stop event of the next GDX_LAUNCH, nullptr outside gdx_numeric
   hipEvent_t launch_ev[2] = {nullptr, nullptr};
   double phase_ms[4] = {0, 0, 0, 0};
