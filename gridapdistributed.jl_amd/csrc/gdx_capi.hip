@@ -484,6 +484,15 @@ int gdx_numeric(gdx_problem *p, int32_t precision) {
   p->precision = precision;
   GDX_HIP(hipSetDevice(p->ctx->device));
   hipStream_t st = p->ctx->stream;
+  // a caller's capture of this stream records the launches alone: nothing runs
+  // now, so the times stay those of the last phase that did
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  GDX_HIP(hipStreamIsCapturing(st, &capturing));
+  if (capturing != hipStreamCaptureStatusNone) {
+    const int rc = gdx::numeric_launches(p, st);
+    if (rc) set_error("numeric kernel launch failed");
+    return rc;
+  }
   for (bool &e : p->ev_set) e = false;
   p->timed = false;
   const bool diffusion = p->desc.op_kind == GDX_OP_DIFFUSION;

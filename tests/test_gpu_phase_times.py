@@ -1,9 +1,13 @@
 """gdx_phase_times on device 0: refused before a numeric phase has run; after one
-of any kind, the stages that launched add up to the total and the others are 0."""
+of any kind, the stages that launched add up to the total and the others are 0.  A
+numeric phase that a caller captures into a graph runs nothing and leaves them."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
-from gridap_amd import flux_operator_from_workload, problem_from_workload
+from gridap_amd import _lib, flux_operator_from_workload, problem_from_workload
 from gridap_amd import workloads as W
 from gridap_amd._lib import GdxError
 
@@ -65,4 +69,48 @@ def test_stages_add_up(gpu_ctx, kind):
     assert 0.0 < t[3] < 1e3 and sum(t[:3]) == pytest.approx(t[3], abs=1e-4)
     for ms, launched in zip(t, KINDS[kind][1]):
         assert launched is None or (ms > 0.0 if launched else ms == 0.0)
+    prob.close()
+
+
+@pytest.mark.parametrize("kind", ["3d cells", "elasticity"])
+def test_capture_of_the_numeric_phase(gpu_ctx, kind):
+    """The numeric phase captured by the program on the library's stream: replays
+    assemble with the coefficient of their time, and no time is taken from it."""
+    prob = problem(gpu_ctx, kind)
+    ncell = int(np.prod(KINDS[kind][0]["cells"]))
+    ptr = ctypes.c_void_p()
+    _lib.call("gdx_stream", prob.handle, ctypes.byref(ptr))
+    stream = torch.cuda.ExternalStream(ptr.value)
+
+    def values():
+        prob.sync()
+        return np.concatenate([np.concatenate([Q["val"], Q["b"]]) for Q in map(prob.export_part, range(prob.nparts))])
+
+    def capture():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(stream):
+            graph.capture_begin(capture_error_mode="thread_local")
+            prob.numeric()
+            graph.capture_end()
+        return graph
+
+    prob.set_cell_coefficient(np.full(ncell, 1.0))
+    graph = capture()
+    refused(prob)  # it has not run
+    prob.numeric()
+    times = prob.phase_times()
+    again = capture()
+    assert prob.phase_times() == times
+    for k, g in enumerate((graph, again, graph)):
+        prob.set_cell_coefficient(np.full(ncell, 2.0 + k))
+        with torch.cuda.stream(stream):
+            g.replay()
+        got = values()
+        prob.set_cell_coefficient(np.full(ncell, 9.0))  # other values in between
+        prob.numeric()
+        prob.sync()
+        prob.set_cell_coefficient(np.full(ncell, 2.0 + k))
+        prob.numeric()
+        assert np.array_equal(got, values())
+    del graph, again
     prob.close()
