@@ -269,6 +269,7 @@ int gdx_problem_create(gdx_ctx *ctx, const gdx_problem_desc *desc, gdx_problem *
   p->D = desc->dim;
   p->K = desc->order;
   p->NQ = desc->qdeg / 2 + 1;
+  if (p->D == 3 && desc->op_kind == GDX_OP_DIFFUSION) p->kvariant3d = 2;
   p->ncomp = desc->op_kind == GDX_OP_ELASTICITY ? 3 : 1;
   p->nparts = p->desc.parts[0] * p->desc.parts[1] * p->desc.parts[2];
   *out = p;

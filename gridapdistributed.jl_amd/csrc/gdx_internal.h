@@ -167,8 +167,8 @@ struct gdx_problem {
   std::vector<gdx::Tile> tiles;
   std::vector<int> tile_pats;
   int n_fast_tiles = 0;  // leading tiles whose position patterns fit in LDS
-  int kvariant3d = 2;    // 3D matrix kernel: 0 z-marching columns, 1 per-tile, 2 pair lattice (the default),
-                         // 3 per-tile wave-slab (Q2)
+  int kvariant3d = 0;    // 3D diffusion's matrix kernel: 0 z-marching columns, 1 per-tile, 2 pair lattice (the
+                         // default), 3 per-tile wave-slab (Q2); 0 for every other problem
   bool hbm_patterns = false;  // every tile takes the HBM-pattern kernel instance (GDX_KERNEL_HBM_PATTERNS)
   int precision = 0;     // contraction precision of the current numeric phase (GDX_PREC_*)
   int tileR[3] = {1, 1, 1};

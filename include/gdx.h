@@ -152,10 +152,12 @@ int gdx_symbolic(gdx_problem *prob);
    (src/Algebra.jl:530-535,755-758).  Ghost rows end with zero values. */
 int gdx_numeric(gdx_problem *prob, int32_t precision);
 
-/* 3D matrix kernel of a problem: variant 0 = z-marching columns with rows_z z
-   rows per workgroup, 1 = per-tile kernel, 2 = pair-lattice kernel (the
+/* 3D matrix kernel of a diffusion problem: variant 0 = z-marching columns with
+   rows_z z rows per workgroup, 1 = per-tile kernel, 2 = pair-lattice kernel (the
    default), 3 = per-tile kernel whose waves own whole rows (Q2 only; rows_z
-   ignored for 1-3).  All give the same matrix to rounding. */
+   ignored for 1-3).  All give the same matrix to rounding.  A 2D problem has one
+   kernel and ignores the choice; gdx_problem_get_kernel gives 0 there and for the
+   other operators. */
 int gdx_problem_set_kernel(gdx_problem *prob, int32_t variant, int32_t rows_z);
 /* variant flag: every tile reads its position patterns from HBM, as the tiles
    with more distinct patterns than the kernel's LDS holds always do (same
@@ -354,10 +356,11 @@ int gdx_fpcg(gdx_problem *prob, gdx_nn *nn, const double *rhs, double rtol, int3
 
 /* Batched numeric assembly: independent problems of uneven sizes and
    partitions (each after gdx_symbolic, all on one context) assembled by one
-   hipGraph launch.  gdx_batch_autotune sets each 3D problem's matrix kernel to
-   the fastest form (chosen, per problem, may be NULL: minus the variant of
-   gdx_problem_set_kernel), which is the pair-lattice kernel at every measured
-   size, so nothing is timed.  gdx_batch_capture records the numeric launches of every problem
+   hipGraph launch.  gdx_batch_autotune sets each 3D diffusion problem's matrix
+   kernel to the pair-lattice kernel, also where the caller had chosen another, and
+   its precision to FP64; nothing is timed (reps, 1 to 100, is checked and not used)
+   (chosen, per problem, may be NULL: minus the variant of gdx_problem_set_kernel, or
+   the z rows per workgroup where that is 0).  gdx_batch_capture records the numeric launches of every problem
    (no memsets) as independent branches of one graph: the problems are spread over four streams
    (largest first, to the least loaded), forked from and joined back into the context's stream, so
    small problems run beside each other; gdx_batch_launch replays the graph on the context's stream

@@ -7,7 +7,7 @@ import pytest
 
 import oracle
 from _helpers import STRUCT_KEYS, rel_err
-from gridap_amd import AssemblyBatch, problem_from_workload
+from gridap_amd import AssemblyBatch, flux_operator_from_workload, problem_from_workload
 from gridap_amd import workloads as W
 from gridap_amd._lib import KERNEL_HBM_PATTERNS
 
@@ -45,6 +45,25 @@ def test_autotuned_tiling_bit_identical(gpu_ctx, p):
             assert rel_err(v1, v0) <= 1e-13 and rel_err(b1, b0) <= 1e-13
     b.close()
     prob.close()
+
+
+def test_kernel_reported_where_there_is_a_choice(gpu_ctx):
+    """Only 3D diffusion has kernels to choose from: the others report variant 0,
+    and the autotuner a positive number."""
+    diffusion = make(gpu_ctx, W.poisson3d_q1(6, (2, 1, 1)))[1]
+    assert diffusion.get_kernel()[0] == 2
+    op = flux_operator_from_workload(gpu_ctx, W.plaplacian3d_q1(6, (2, 1, 1)))
+    others = [make(gpu_ctx, W.poisson2d_q1(8, (2, 1)))[1], op._problem(),
+              make(gpu_ctx, W.elasticity3d_q2((3, 3, 2), (1, 1, 1)))[1]]
+    assert [prob.get_kernel()[0] for prob in others] == [0, 0, 0]
+    b = AssemblyBatch(gpu_ctx)
+    for prob in [diffusion] + others:
+        b.add(prob)
+    chosen = b.autotune(reps=1)
+    assert chosen[0] == -2 and all(c > 0 for c in chosen[1:])
+    b.close()
+    for prob in [diffusion] + others:
+        prob.close()
 
 
 @pytest.mark.parametrize("p", [W.poisson3d_q2_fourier(9, (2, 1, 3)), W.poisson3d_q2_fourier(6, (1, 2, 2), strategy="full"),
