@@ -1205,14 +1205,14 @@ int mg_setup(TwoGrid *T, hipStream_t st) {
       const size_t v = (size_t)L.m * L.m * L.m;
       T->lv.push_back(L);
       Level &M = T->lv.back();
-      bool ok = hipMalloc(reinterpret_cast<void **>(&M.rhs), v * sizeof(double)) == hipSuccess &&
-                hipMalloc(reinterpret_cast<void **>(&M.e), v * sizeof(double)) == hipSuccess &&
-                hipMalloc(reinterpret_cast<void **>(&M.e2), v * sizeof(double)) == hipSuccess;
+      bool ok = dev_malloc(reinterpret_cast<void **>(&M.rhs), v * sizeof(double)) == hipSuccess &&
+                dev_malloc(reinterpret_cast<void **>(&M.e), v * sizeof(double)) == hipSuccess &&
+                dev_malloc(reinterpret_cast<void **>(&M.e2), v * sizeof(double)) == hipSuccess;
       if (l == 0) {
         M.cst = T->cst;
         M.own_cst = false;
       } else {
-        ok = ok && hipMalloc(reinterpret_cast<void **>(&M.cst), 27 * v * sizeof(double)) == hipSuccess;
+        ok = ok && dev_malloc(reinterpret_cast<void **>(&M.cst), 27 * v * sizeof(double)) == hipSuccess;
       }
       if (!ok) {
         mg_free(T);
@@ -1351,15 +1351,9 @@ static int fine_stencil(TwoGrid *T, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 
-// bind the network to a problem's current matrix: transfer maps, the fine
-// inverse diagonal on the lattice and the network's diagonal feature
-int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
+static int attach(gdx_nn *nn, gdx_problem *p) {
   nn::Net &N = nn->net;
   const int n = N.n;
-  if (p->D != 3 || p->K != 1) return GDX_ERR_UNSUPPORTED;
-  if (p->desc.dir_kind != 1) return GDX_ERR_UNSUPPORTED;
-  for (int d = 0; d < 3; ++d)
-    if (p->kp.ncells[d] != 2 * n) return GDX_ERR_ARG;
   hipStream_t st = p->ctx->stream;
   TwoGrid *T = tg_of(nn);
   if (T && T->prob != p) {
@@ -1387,27 +1381,24 @@ int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
         gid_node[P.ldof_gid[i]] = g0 + (int64_t)nf * (g1 + (int64_t)nf * g2);
       }
     const size_t gsz = std::max<int64_t>(p->ngdofs, 1) * sizeof(double);
-    bool ok = hipMalloc(reinterpret_cast<void **>(&T->gid_node), std::max<int64_t>(p->ngdofs, 1) * sizeof(long long)) ==
+    bool ok = dev_malloc(reinterpret_cast<void **>(&T->gid_node), std::max<int64_t>(p->ngdofs, 1) * sizeof(long long)) ==
                   hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->flat), nfl * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->dlat), nfl * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->t1), gsz) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->t2), gsz) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->t3), gsz) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->rho), v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->red), (kS + 16) * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->ec), v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->ec2), v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->tgt), v * sizeof(float)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->fst), 27 * nfl * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->cst), 27 * v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->rc), v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->ca), v * sizeof(double)) == hipSuccess &&
-              hipMalloc(reinterpret_cast<void **>(&T->cb), v * sizeof(double)) == hipSuccess;
-    if (!ok) {
-      twogrid_free(nn);
-      return GDX_ERR_ALLOC;
-    }
+              dev_malloc(reinterpret_cast<void **>(&T->flat), nfl * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->dlat), nfl * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->t1), gsz) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->t2), gsz) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->t3), gsz) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->rho), v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->red), (kS + 16) * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->ec), v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->ec2), v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->tgt), v * sizeof(float)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->fst), 27 * nfl * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->cst), 27 * v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->rc), v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->ca), v * sizeof(double)) == hipSuccess &&
+              dev_malloc(reinterpret_cast<void **>(&T->cb), v * sizeof(double)) == hipSuccess;
+    if (!ok) return GDX_ERR_ALLOC;
     // the entries of absent neighbours stay zero: one matrix pattern for as long as the attachment lasts
     if (hipMemsetAsync(T->fst, 0, 27 * nfl * sizeof(double), st) != hipSuccess) return GDX_ERR_HIP;
     if (p->dev_numbering ? gid_node_device(p, T->gid_node) != GDX_OK
@@ -1426,6 +1417,23 @@ int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
   galerkin(n, nf, 0, nfl, T->fst, T->cst, st);
   if ((rc = mg_setup(T, st))) return rc;
   return hipStreamSynchronize(st) == hipSuccess ? GDX_OK : GDX_ERR_HIP;
+}
+
+// bind the network to a problem's current matrix: transfer maps, the fine
+// inverse diagonal on the lattice and the network's diagonal feature.  A binding
+// that fails half way is dropped: the next one to the same problem starts anew.
+int twogrid_attach(gdx_nn *nn, gdx_problem *p) {
+  if (p->D != 3 || p->K != 1) return GDX_ERR_UNSUPPORTED;
+  if (p->desc.dir_kind != 1) return GDX_ERR_UNSUPPORTED;
+  for (int d = 0; d < 3; ++d)
+    if (p->kp.ncells[d] != 2 * nn->net.n) return GDX_ERR_ARG;
+  const int rc = attach(nn, p);
+  if (rc) {
+    (void)hipStreamSynchronize(p->ctx->stream);
+    (void)hipGetLastError();  // an allocation's, seen already
+    twogrid_free(nn);
+  }
+  return rc;
 }
 
 // the coarse correction of the fine residual s (global-id order, or on the
@@ -1703,6 +1711,7 @@ int gdx_nn_attach(gdx_nn *nn, gdx_problem *prob) {
     return GDX_ERR_ARG;
   }
   if (hipSetDevice(prob->ctx->device) != hipSuccess) return GDX_ERR_HIP;
+  const gdx::FaultScope fault_scope;
   int rc = gdx::twogrid_attach(nn, prob);
   if (rc == GDX_ERR_UNSUPPORTED) gdx::set_error("the two-grid preconditioner is built for 3D Q1 with Dirichlet data on the whole boundary");
   else if (rc == GDX_ERR_ARG) gdx::set_error("the problem must have 2n x 2n x 2n cells for a network grid of n^3");

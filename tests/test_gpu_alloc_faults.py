@@ -7,13 +7,15 @@ the call returns GDX_ERR_ALLOC, the problem refuses a numeric phase
 assembles exactly what a problem that never failed assembles.  Covers the
 device numbering, CSR, pattern, row-table and tile stages, the buffers
 gdx_symbolic allocates after them, and the flux and elasticity set-ups.
+
+The same for gdx_nn_attach: a binding that fails half way is dropped.
 """
 import os
 
 import numpy as np
 import pytest
 
-from gridap_amd import fespaces, problem_from_workload
+from gridap_amd import LearnedCoarseSolver, fespaces, fpcg, problem_from_workload
 from gridap_amd import workloads as W
 from gridap_amd._lib import GdxError
 
@@ -76,3 +78,43 @@ def test_every_failed_allocation_is_reported_and_recoverable(gpu_ctx, p):
         assert n < 500
     print("device allocations in the symbolic phase:", n, flush=True)
     assert n >= 20
+
+
+def test_failed_attach_is_dropped(gpu_ctx):
+    print("allocation faults in gdx_nn_attach", flush=True)
+    assem, data = problem_from_workload(gpu_ctx, W.poisson3d_q1(16, (2, 1, 1)))
+    prob = assem._problem_for(data)
+    prob.numeric()
+    prob.sync()
+    rhs = np.random.default_rng(0).normal(size=prob.ngdofs)
+    net = LearnedCoarseSolver(gpu_ctx, 8, 1)
+    net.attach(prob)
+    net.set_options(2, use_network=False)
+    ref = fpcg(prob, net, rhs, 1e-10)[0]
+    net.close()
+    n = 0
+    while True:
+        net = LearnedCoarseSolver(gpu_ctx, 8, 1)
+        os.environ["GDX_FAULT_ALLOC"] = str(n)
+        try:
+            net.attach(prob)
+            failed = False
+        except GdxError as e:
+            assert e.code == ERR_ALLOC, (n, e)
+            failed = True
+        finally:
+            os.environ.pop("GDX_FAULT_ALLOC", None)
+        if failed:
+            with pytest.raises(GdxError) as e:
+                net.apply(rhs)
+            assert e.value.code == ERR_STATE, n
+            net.attach(prob)
+        net.set_options(2, use_network=False)
+        assert np.array_equal(fpcg(prob, net, rhs, 1e-10)[0], ref), n
+        net.close()
+        if not failed:
+            break
+        n += 1
+        assert n < 100
+    assert n >= 16 + 3  # the attachment's buffers and at least a level's
+    prob.close()
