@@ -224,9 +224,9 @@ void unregister(std::vector<T *> &v, T *x) {
     }
 }
 int symbolic(gdx_problem *p);  // symbolic phase (gdx_symbolic.cpp)
-// The device allocations of the symbolic phase and of gdx_nn_attach go through
-// dev_malloc: it is hipMalloc, except that GDX_FAULT_ALLOC=n, read when such a
-// call starts (FaultScope), makes the n-th of that call's allocations (from 0) fail as
+// The device allocations of the symbolic phase, of gdx_nn_attach and of gdx_fpcg's
+// lattice vectors go through dev_malloc: it is hipMalloc, except that
+// GDX_FAULT_ALLOC=n, read when such a call starts (FaultScope), makes the n-th of that call's allocations (from 0) fail as
 // exhausted HBM would, once, so that the error paths can be tested.
 hipError_t dev_malloc(void **p, size_t bytes);
 template <class T>

@@ -1601,7 +1601,7 @@ FpcgPrec twogrid_prec(gdx_nn *nn, bool current) {
   TwoGrid *T = tg_of(nn);
   const int64_t nfl = T ? (int64_t)T->nf * T->nf * T->nf : 0;
   if (!T || nfl >= (int64_t)1 << 30) return p;  // 32-bit node ids in the kernels
-  if (!T->lat && hipMalloc(reinterpret_cast<void **>(&T->lat), (kLcount * nfl + 2 * nb(nfl) + 1) * sizeof(double)) !=
+  if (!T->lat && dev_malloc(reinterpret_cast<void **>(&T->lat), (kLcount * nfl + 2 * nb(nfl) + 1) * sizeof(double)) !=
                      hipSuccess) {
     (void)hipGetLastError();
     T->lat = nullptr;  // no room: the products from the CSR rows, in global-id order
@@ -1870,6 +1870,7 @@ int gdx_fpcg(gdx_problem *prob, gdx_nn *nn, const double *rhs, double rtol, int3
     return GDX_ERR_STATE;
   }
   if (hipSetDevice(prob->ctx->device) != hipSuccess) return GDX_ERR_HIP;
+  const gdx::FaultScope fault_scope;
   const gdx::FpcgPrec pr = nn ? gdx::twogrid_prec(nn, false) : gdx::FpcgPrec{};
   int it = 0, fb = 0;
   int rc = gdx::solve_fpcg(prob, nn ? &pr : nullptr, rhs, rtol, maxiter, xsol, &it, relres, ms, &fb);

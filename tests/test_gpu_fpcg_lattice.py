@@ -73,6 +73,34 @@ def test_fpcg_on_the_lattice_matches_direct_solve(gpu_ctx, cells, parts, factor)
     prob.close()
 
 
+@pytest.mark.parametrize("use_network", [False, True])
+def test_fpcg_without_room_for_the_lattice_vectors(gpu_ctx, monkeypatch, use_network):
+    """Where the lattice vectors do not fit the iteration runs in global-id order, its
+    products on the CSR rows; the next solve finds room again."""
+    assem, data = problem_from_workload(gpu_ctx, W.poisson3d_q1(16, (2, 1, 2), rhs_const=0.0))
+    prob = assem._problem_for(data)
+    prob.cell_coefficient_grf(3, 0.1, 2.0)
+    prob.numeric()
+    prob.sync()
+    net = LearnedCoarseSolver(gpu_ctx, 8, 1)
+    net.attach(prob)
+    net.set_options(2, use_network=use_network)
+    A = matrix(prob, 4)
+    rhs = np.random.default_rng(2).normal(size=prob.ngdofs)
+    ref = spl.spsolve(A, rhs)
+    monkeypatch.setenv("GDX_FAULT_ALLOC", "0")
+    ids, it0, relres0, _, fb0 = fpcg(prob, net, rhs, 1e-10)
+    monkeypatch.delenv("GDX_FAULT_ALLOC")
+    lattice, it1, relres1, _, fb1 = fpcg(prob, net, rhs, 1e-10)
+    for x, relres, fb in ((ids, relres0, fb0), (lattice, relres1, fb1)):
+        assert not fb and relres <= 1.01e-10
+        assert np.linalg.norm(x - ref) <= 1e-6 * np.linalg.norm(ref)
+    assert abs(it0 - it1) <= 1
+    assert not np.array_equal(ids, lattice)  # two iterations: their sums run in different orders
+    net.close()
+    prob.close()
+
+
 # networks of 8 to 40 cells: a level of three to seven cells at the bottom (one
 # wave up to five, else a workgroup), levels that the 16 x 2 x 2 and 16 x 4 x 4
 # node tiles do not divide, and one above 32 whose residual is a launch of its own
