@@ -601,22 +601,29 @@ struct ShapeOf<2, 1, NQ> {
   using type = LatShape<2, 1, NQ, 16, 16, 1, 256, 16>;
 };
 
-// row table on the global lattice, padded to whole tiles, from the parts' tables
+// row table on the global lattice, padded to whole tiles, from the parts' tables.
+// A grid holds 65535 blocks in y and in z (a long box has more lines): each takes
+// every gridDim-th line there.
+constexpr int kLatRowsGrid = 32768;
 template <int K>
 __global__ void k_lat_rows(LatArgs a, int parts0, int parts1, const int *__restrict__ node_part,
                            const LatPart *__restrict__ parts, const RowInfo *__restrict__ rowinfo,
                            LatRow *__restrict__ rows) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
+  const int x = blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= a.pn[0]) return;
-  LatRow r{0, 0, -1};
-  if (x < a.nn[0] && y < a.nn[1] && z < a.nn[2]) {
-    const LatPart P =
-        parts[node_part[x] + parts0 * (node_part[a.nn[0] + y] + parts1 * node_part[a.nn[0] + a.nn[1] + z])];
-    const RowInfo ri = rowinfo[P.base + ((long long)(z - P.lo[2]) * P.n[1] + (y - P.lo[1])) * P.n[0] + (x - P.lo[0])];
-    if (ri.pid >= 0)
-      r = LatRow{8 * ri.rowstart, ri.pid << 9 | ((ri.lenf >> 16) & 1) << 8 | (ri.lenf & 0xFF), (int)ri.bidx};
-  }
-  rows[row_at<K>(a, x, y, z)] = r;
+  for (int z = blockIdx.z; z < a.pn[2]; z += gridDim.z)
+    for (int y = blockIdx.y; y < a.pn[1]; y += gridDim.y) {
+      LatRow r{0, 0, -1};
+      if (x < a.nn[0] && y < a.nn[1] && z < a.nn[2]) {
+        const LatPart P =
+            parts[node_part[x] + parts0 * (node_part[a.nn[0] + y] + parts1 * node_part[a.nn[0] + a.nn[1] + z])];
+        const RowInfo ri =
+            rowinfo[P.base + ((long long)(z - P.lo[2]) * P.n[1] + (y - P.lo[1])) * P.n[0] + (x - P.lo[0])];
+        if (ri.pid >= 0)
+          r = LatRow{8 * ri.rowstart, ri.pid << 9 | ((ri.lenf >> 16) & 1) << 8 | (ri.lenf & 0xFF), (int)ri.bidx};
+      }
+      rows[row_at<K>(a, x, y, z)] = r;
+    }
 }
 
 struct LatData {
@@ -833,7 +840,7 @@ int lattice_setup(gdx_problem *p) {
   const int *node_part = reinterpret_cast<const int *>(dtab + at_np);
   if (!rc) {
     hipStream_t st = p->ctx->stream;
-    const dim3 g((a.pn[0] + 255) / 256, a.pn[1], a.pn[2]);
+    const dim3 g((a.pn[0] + 255) / 256, std::min(a.pn[1], kLatRowsGrid), std::min(a.pn[2], kLatRowsGrid));
     const auto kernel = K == 2 ? k_lat_rows<2> : k_lat_rows<1>;
     hipLaunchKernelGGL(kernel, g, dim3(256), 0, st, a, p->desc.parts[0], p->desc.parts[1], node_part, dparts,
                        p->dev.rowinfo, L->rows);
