@@ -48,7 +48,6 @@
 #include <vector>
 
 #include "gdx_internal.h"
-#include "gdx_launch.h"
 
 namespace gdx {
 
@@ -501,7 +500,7 @@ int elast_assemble(gdx_problem *p, hipStream_t st) {
     const double *coef = p->coef_cell ? p->dev.cellk : p->dev.cell_lame;
     if (!coef) return GDX_ERR_STATE;
 #define GDX_ELAST_CW(KK, CW)                                                                                       \
-  GDX_LAUNCH(p, (k_elast_cw<KK, kNodesPerWave, CW>), grid, block, st, A, E->rows, E->sfac, E->sinfo, coef, \
+  hipLaunchKernelGGL((k_elast_cw<KK, kNodesPerWave, CW>), grid, block, 0, st, A, E->rows, E->sfac, E->sinfo, coef, \
                      E->mass, E->pinv, p->dev.values, p->dev.b)
     if (p->K == 2 && p->coef_cell) GDX_ELAST_CW(2, 1);
     else if (p->K == 2) GDX_ELAST_CW(2, 2);
@@ -511,10 +510,10 @@ int elast_assemble(gdx_problem *p, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
   }
   if (p->K == 2)
-    GDX_LAUNCH(p, (k_elast<2, kNodesPerWave>), grid, block, st, A, E->rows, E->fac, E->mass, E->pinv,
+    hipLaunchKernelGGL((k_elast<2, kNodesPerWave>), grid, block, 0, st, A, E->rows, E->fac, E->mass, E->pinv,
                        p->dev.values, p->dev.b);
   else
-    GDX_LAUNCH(p, (k_elast<1, kNodesPerWave>), grid, block, st, A, E->rows, E->fac, E->mass, E->pinv,
+    hipLaunchKernelGGL((k_elast<1, kNodesPerWave>), grid, block, 0, st, A, E->rows, E->fac, E->mass, E->pinv,
                        p->dev.values, p->dev.b);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }

@@ -183,13 +183,11 @@ struct gdx_problem {
   gdx::DevNumbering dn;
   gdx::KParams kp{};
   gdx::Device dev;
-  // timing of the last numeric phase: start of its first kernel, ends of the
-  // coefficient, RHS and matrix stages (ev_set: the stages that launched)
-  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-  bool ev_set[4] = {false, false, false, false};
+  // timing of the last numeric phase: the device clock at its start and at the ends
+  // of the coefficient, RHS and matrix stages (stamped: the stages that launched)
+  unsigned long long *stamps = nullptr;  // [4], device
+  bool stamped[4] = {false, false, false, false};
   bool timed = false;  // a numeric phase has run (and the last one did not fail)
-  // start and stop event of the next GDX_LAUNCH, nullptr outside gdx_numeric
-  hipEvent_t launch_ev[2] = {nullptr, nullptr};
   double phase_ms[4] = {0, 0, 0, 0};
   void *solve = nullptr;  // solver state (gdx_solve.hip), built on the first solve
   void *flux = nullptr;   // nonlinear operator state (gdx_flux.hip)

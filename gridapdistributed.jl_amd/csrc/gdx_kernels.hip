@@ -26,7 +26,6 @@
 #include <vector>
 
 #include "gdx_device.h"
-#include "gdx_launch.h"
 
 namespace gdx {
 
@@ -204,18 +203,14 @@ int launch_coefficients(gdx_problem *p, hipStream_t st) {
   const int qnmax = longest_line(kp);
   if (kp.nmodes > 0) {
     dim3 g1((qnmax + 255) / 256, kp.nmodes, 3);
-    const hipEvent_t stop = p->launch_ev[1];
-    p->launch_ev[1] = nullptr;
-    GDX_LAUNCH(p, k_fourier_tables, g1, dim3(256), st, p->dev.modes, kp, qnmax, p->dev.E);
-    p->launch_ev[0] = nullptr;
-    p->launch_ev[1] = stop;
+    hipLaunchKernelGGL(k_fourier_tables, g1, dim3(256), 0, st, p->dev.modes, kp, qnmax, p->dev.E);
   }
   const int bx = kp.qn[0] < 256 ? 64 * ((kp.qn[0] + 63) / 64) : 256;
   dim3 g2((kp.qn[0] + bx - 1) / bx, (kp.qn[1] + kCoefLines - 1) / kCoefLines, kp.qn[2]);
   const bool source = kp.rhs_kind == GDX_RHS_MANUFACTURED, few = kp.nmodes <= 8;
   const auto kernel = source ? (few ? k_coefficients<true, 8> : k_coefficients<true, 16>)
                              : (few ? k_coefficients<false, 8> : k_coefficients<false, 16>);
-  GDX_LAUNCH(p, kernel, g2, dim3(bx), st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, source_array(p));
+  hipLaunchKernelGGL(kernel, g2, dim3(bx), 0, st, p->dev.modes, p->dev.E, kp, qnmax, p->dev.W, source_array(p));
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 

@@ -36,7 +36,6 @@
 #include <vector>
 
 #include "gdx_device.h"
-#include "gdx_launch.h"
 #include "gdx_lattice.h"
 
 namespace gdx {
@@ -568,7 +567,7 @@ void launch_source(gdx_problem *p, const LatArgs &a, const double *F, hipStream_
   constexpr int R[3] = {16, D == 3 ? 8 : 16, D == 3 ? 4 : 1};
   dim3 g((a.hi[0] - a.lo[0] + R[0] - 1) / R[0], (a.hi[1] - a.lo[1] + R[1] - 1) / R[1],
          (a.hi[2] - a.lo[2] + R[2] - 1) / R[2]);
-  if (g.x && g.y && g.z) GDX_LAUNCH(p, (k_source<D, K, NQ>), g, dim3(256), st, a, F);
+  if (g.x && g.y && g.z) hipLaunchKernelGGL((k_source<D, K, NQ>), g, dim3(256), 0, st, a, F);
 }
 
 template <int D, int K, int NQ>
@@ -691,7 +690,7 @@ template <class T>
 int launch(gdx_problem *p, LatArgs &a, hipStream_t st) {
   const int64_t n = cut_tiles<T>(a), lines = n / a.nt[0];
   const int64_t grid = 8 * ((lines + 7) / 8) * a.nt[0];
-  GDX_LAUNCH(p, (k_lattice<T>), dim3((unsigned)grid), dim3(T::NT), st, a, (int)n);
+  hipLaunchKernelGGL((k_lattice<T>), dim3((unsigned)grid), dim3(T::NT), 0, st, a, (int)n);
   return hipGetLastError() == hipSuccess ? GDX_OK : GDX_ERR_HIP;
 }
 

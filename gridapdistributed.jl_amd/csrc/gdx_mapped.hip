@@ -30,7 +30,6 @@
 #include <vector>
 
 #include "gdx_internal.h"
-#include "gdx_launch.h"
 
 namespace gdx {
 
@@ -515,17 +514,19 @@ int launch_mapped_t(gdx_problem *p, MappedData *M, hipStream_t st, bool rows_sta
     // take every (WPB x workgroups)-th cell
     const long long blocks = std::min<long long>((M->ncell + WPB - 1) / WPB, kMappedBlocks);
     if (p->reac_w != 0.0)
-      GDX_LAUNCH(p, (k_mapped_cells<D, K, NQ, true>), dim3((unsigned)std::max<long long>(blocks, 1)), dim3(64 * WPB), st, p->kp, M->ncell, M->vc, p->dev.modes,
+      hipLaunchKernelGGL((k_mapped_cells<D, K, NQ, true>), dim3((unsigned)std::max<long long>(blocks, 1)),
+                         dim3(64 * WPB), 0, st, p->kp, M->ncell, M->vc, p->dev.modes,
                          p->coef_cell ? p->dev.cellk : nullptr, p->diff_w, p->reac_w, M->cm);
     else
-      GDX_LAUNCH(p, (k_mapped_cells<D, K, NQ, false>), dim3((unsigned)std::max<long long>(blocks, 1)), dim3(64 * WPB), st, p->kp, M->ncell, M->vc, p->dev.modes,
+      hipLaunchKernelGGL((k_mapped_cells<D, K, NQ, false>), dim3((unsigned)std::max<long long>(blocks, 1)),
+                         dim3(64 * WPB), 0, st, p->kp, M->ncell, M->vc, p->dev.modes,
                          p->coef_cell ? p->dev.cellk : nullptr, p->diff_w, 0.0, M->cm);
   } else if (M->nrows > 0) {
     constexpr int LPR = Sh::S <= 16 ? 16 : (Sh::S <= 32 ? 32 : 64);
     const long long groups = (M->nrows + kMappedRowsPerGroup - 1) / kMappedRowsPerGroup;
     const long long blocks = ((groups * LPR + 255) / 256 + 7) / 8 * 8;  // a multiple of 8 (XCD order)
     if (blocks > 0x7FFFFFFFLL) return GDX_ERR_UNSUPPORTED;
-    GDX_LAUNCH(p, (k_mapped_rows<D, K, kMappedRowsPerGroup>), dim3((unsigned)blocks), dim3(256), st, p->kp,
+    hipLaunchKernelGGL((k_mapped_rows<D, K, kMappedRowsPerGroup>), dim3((unsigned)blocks), dim3(256), 0, st, p->kp,
                        M->nrows, M->rows,
                        p->dev.pat_fwd, pattern_stride(p->kp.S), M->cm, M->vc, p->dev.values, p->dev.b);
   }

@@ -415,8 +415,10 @@ int gdx_psparse_mul(gdx_problem *prob, gdx_pvector *y, gdx_pvector *x);
 int gdx_device_values(gdx_problem *prob, double **values, int64_t *nnz_total);
 int gdx_stream(gdx_problem *prob, void **stream);
 int gdx_sync(gdx_problem *prob);
-/* per-phase device times (ms) of the last gdx_numeric, measured with hipEvents
-   on the library's stream: [0] coefficient, [1] rhs, [2] matrix, [3] total */
+/* per-phase device times (ms) of the last gdx_numeric, from the device clock read
+   between the stages on the stream: [0] coefficient, [1] rhs, [2] matrix, [3] total
+   (0: the stage launched nothing); waits for the stream.  GDX_ERR_STATE before a
+   numeric phase has run.  A gdx_numeric that a caller captures is not timed. */
 int gdx_phase_times(gdx_problem *prob, double *ms, int32_t n);
 /* number of owned free x free stored entries (the Gnnz/s numerator) */
 int gdx_owned_nnz(gdx_problem *prob, int64_t *nnz);
