@@ -47,7 +47,7 @@ def test_kernel_change_drops_the_graph(gpu_ctx):
     b2.capture()
     b1.launch()
     b1.sync()
-    prob.set_kernel(2)  # re-uploads the tiles and row table of prob
+    prob.set_kernel(0, 8)  # makes and uploads prob's tiles and pattern lists anew
     launch_state_error(b1)
     b2.launch()  # a batch without prob keeps its graph
     b2.sync()
@@ -58,6 +58,8 @@ def test_kernel_change_drops_the_graph(gpu_ctx):
     prob.numeric()
     for (v0, c0), (v1, c1) in zip(ref, values(prob)):
         assert np.array_equal(v0, v1) and np.array_equal(c0, c1)
+    prob.set_kernel(2)  # no tiles, but another kernel than the captured one
+    launch_state_error(b1)
     for x in (b1, b2, prob, other):
         x.close()
 
