@@ -2,10 +2,10 @@
 // sizes and partitions) assembled by one graph launch.
 //
 //   gdx_batch_add       problems after their symbolic phase, on one context
-//   gdx_batch_autotune  sets every 3D problem's matrix kernel to the pair-lattice
-//                       kernel, the fastest form at every size: 3D Q2 64^3 0.42 ms
+//   gdx_batch_autotune  sets every 3D diffusion problem's matrix kernel to the
+//                       pair-lattice kernel and times nothing: 3D Q2 64^3 0.42 ms
 //                       against 0.79 (z-marching) and 0.63 (per tile); Q1
-//                       131 x 97 x 75 0.050 ms against 0.45
+//                       131 x 97 x 75 0.050 ms against 0.45 (z-marching)
 //   gdx_batch_capture   records every problem's numeric launches (coefficient,
 //                       RHS and matrix kernels; no memsets) into one hipGraph:
 //                       the diffusion problems on the uniform box go together,

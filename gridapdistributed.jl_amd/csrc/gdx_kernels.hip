@@ -14,12 +14,14 @@
 // entry int_c kappa grad(phi_i).grad(phi_j) for the affine Cartesian map
 // (J = diag(h), detJ = h1 h2 h3, J^{-T} grad = grad_ref / h).  The three
 // contractions over x-, y- and z-quadrature points are done one dimension at
-// a time in LDS (sum factorisation), so each stored value costs O(1) FMAs.
-// Rows are staged in LDS and written once, contiguously, through a position
-// pattern (stencil slot -> offset within the CSR row), so the scatter is a
-// plain coalesced store: no float atomics, bit-for-bit repeatable.  The
+// a time (sum factorisation), so each stored value costs O(1) FMAs.  Every row is
+// written once, contiguously, through a position pattern (stencil slot <-> offset
+// within the CSR row): no float atomics, bit-for-bit repeatable.  The
 // SubAssembledRows owner/ghost exchange is folded in: owned rows receive the
 // neighbouring parts' contributions at the source, ghost rows stay zero.
+// The matrix kernels are in gdx_lattice.hip (the default), gdx_march3d.hip and
+// gdx_tile3d.hip; this file has the coefficients at the quadrature points and the
+// numeric phase's launchers.
 #include <hip/hip_runtime.h>
 
 #include <new>
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(64) void k_coefficients_batch(const CoefProblem *__
 }
 
 // ---------------------------------------------------------------------------
-// launchers.  Tile shapes here must match tile_shape() in gdx_symbolic.cpp.
+// launchers
 // ---------------------------------------------------------------------------
 static int longest_line(const KParams &kp) {
   int qnmax = kp.qn[0];

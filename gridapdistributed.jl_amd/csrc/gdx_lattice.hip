@@ -22,8 +22,8 @@
 //
 // Measured against the z-marching kernel that was the default before, whole
 // numeric phases: 3D Q2 64^3, Fourier kappa 0.86 -> 0.51 ms (the matrix kernel
-// 790 -> 410 us); 3D Q1 131 x 97 x 75, kappa per cell 517 -> 70 us (453 -> 50);
-// 2D Q1 256^2 95 -> 18 us (71 -> 9).  The Q2 kernel writes 2.4 TB/s of the 6.7
+// 790 -> 410 us); 3D Q1 131 x 97 x 75, kappa per cell 517 -> 69 us (453 -> 50);
+// 2D Q1 256^2 95 -> 13 us (71 -> 9).  The Q2 kernel writes 2.4 TB/s of the 6.7
 // that a fill reaches; what is left is latency: at two workgroups per CU the
 // LDS contraction (about 40% of a tile's time) hides behind little else.
 //

@@ -360,11 +360,15 @@ int gdx_fpcg(gdx_problem *prob, gdx_nn *nn, const double *rhs, double rtol, int3
    kernel to the pair-lattice kernel, also where the caller had chosen another, and
    its precision to FP64; nothing is timed (reps, 1 to 100, is checked and not used)
    (chosen, per problem, may be NULL: minus the variant of gdx_problem_set_kernel, or
-   the z rows per workgroup where that is 0).  gdx_batch_capture records the numeric launches of every problem
-   (no memsets) as independent branches of one graph: the problems are spread over four streams
-   (largest first, to the least loaded), forked from and joined back into the context's stream, so
-   small problems run beside each other; gdx_batch_launch replays the graph on the context's stream
-   and the results equal separate gdx_numeric calls bit for bit.
+   the z rows per workgroup where that is 0).  gdx_batch_capture records the numeric
+   launches of every problem (no memsets) in one graph.  The diffusion problems on the
+   uniform box that take the pair-lattice kernel go together, on the context's stream:
+   two launches for all coefficients at quadrature points, a launch per varying source,
+   one per tile shape for the matrices.  The others are independent branches over four
+   streams (largest first, to the least loaded), forked from and joined back into the
+   context's stream, so small problems run beside each other.  gdx_batch_launch replays
+   the graph on the context's stream and the results equal separate gdx_numeric calls
+   bit for bit.
    The reference has no counterpart: it assembles one problem per call
    (src/FESpaces.jl:785-798). */
 typedef struct gdx_batch gdx_batch;
