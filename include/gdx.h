@@ -161,7 +161,8 @@ int gdx_numeric(gdx_problem *prob, int32_t precision);
 int gdx_problem_set_kernel(gdx_problem *prob, int32_t variant, int32_t rows_z);
 /* variant flag: every tile reads its position patterns from HBM, as the tiles
    with more distinct patterns than the kernel's LDS holds always do (same
-   values; lets tests run those kernel instances on small meshes) */
+   values; lets tests run those kernel instances on small meshes).  The pair-lattice
+   kernel has no such tiles and ignores it. */
 #define GDX_KERNEL_HBM_PATTERNS 0x100
 int gdx_problem_get_kernel(gdx_problem *prob, int32_t *variant, int32_t *rows_z);
 
