@@ -31,6 +31,9 @@ struct gdx_batch {
   // the diffusion problems on the uniform box, together in a few launches
   gdx::LatticeBatch *lattice = nullptr;
   gdx::CoefBatch *coef = nullptr;
+  // tables of dropped graphs, not yet freed
+  std::vector<gdx::LatticeBatch *> old_lattice;
+  std::vector<gdx::CoefBatch *> old_coef;
   // capture-time fork/join streams and events (default priority)
   std::vector<hipStream_t> side;
   std::vector<hipEvent_t> ev;  // [0] fork, [1..] joins
@@ -73,13 +76,23 @@ void drop_graph(gdx_batch *b) {
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->exec = nullptr;
   b->graph = nullptr;
-  if (b->lattice || b->coef) {  // a replay in flight reads the tables
-    if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
-    gdx::lattice_batch_free(b->lattice);
-    gdx::coef_batch_free(b->coef);
-    b->lattice = nullptr;
-    b->coef = nullptr;
+  if (b->lattice) b->old_lattice.push_back(b->lattice);
+  if (b->coef) b->old_coef.push_back(b->coef);
+  b->lattice = nullptr;
+  b->coef = nullptr;
+  if (b->old_lattice.empty() && b->old_coef.empty()) return;
+  // a replay in flight reads the tables; while a caller captures the stream it can
+  // neither be waited for nor memory freed, and they stay until the next time
+  if (b->ctx) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(b->ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
+      return;
+    (void)hipStreamSynchronize(b->ctx->stream);
   }
+  for (gdx::LatticeBatch *t : b->old_lattice) gdx::lattice_batch_free(t);
+  for (gdx::CoefBatch *t : b->old_coef) gdx::coef_batch_free(t);
+  b->old_lattice.clear();
+  b->old_coef.clear();
 }
 
 }  // namespace

@@ -8,10 +8,13 @@ instead of replaying freed memory.  Flux problems get their device state in
 gdx_symbolic, so a batch captured right after it records only kernel launches
 and replays the eager numeric phase bit for bit.
 """
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
-from gridap_amd import AssemblyBatch, flux_operator_from_workload, problem_from_workload
+from gridap_amd import _lib, AssemblyBatch, flux_operator_from_workload, problem_from_workload
 from gridap_amd import workloads as W
 from gridap_amd._lib import GdxError
 
@@ -88,6 +91,41 @@ def test_coefficient_mode_and_precision_drop_the_graph(gpu_ctx):
     b.capture()
     prob.symbolic()  # device buffers re-made
     launch_state_error(b)
+    b.close()
+    prob.close()
+
+
+def test_graph_dropped_inside_a_callers_capture(gpu_ctx):
+    """A numeric phase in another precision drops the batch's graph also where the
+    caller is capturing the stream, which then can neither wait nor free."""
+    prob = make(gpu_ctx, W.poisson3d_q1(8, (2, 1, 1)))
+    prob.numeric(1)
+    ref = values(prob)
+    prob.numeric(0)
+    prob.sync()
+    b = AssemblyBatch(gpu_ctx)
+    b.add(prob)
+    b.capture()
+    b.launch()
+    b.sync()
+    ptr = ctypes.c_void_p()
+    _lib.call("gdx_stream", prob.handle, ctypes.byref(ptr))
+    stream, graph = torch.cuda.ExternalStream(ptr.value), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        graph.capture_begin(capture_error_mode="thread_local")
+        try:
+            prob.numeric(1)
+        finally:
+            graph.capture_end()
+    launch_state_error(b)
+    with torch.cuda.stream(stream):
+        graph.replay()
+    for (v0, c0), (v1, c1) in zip(ref, values(prob)):
+        assert np.array_equal(v0, v1) and np.array_equal(c0, c1)
+    b.capture()  # and frees what the dropped graph had used
+    b.launch()
+    b.sync()
+    del graph
     b.close()
     prob.close()
 
